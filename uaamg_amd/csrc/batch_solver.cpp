@@ -365,7 +365,6 @@ int PoissonBatch::init(std::vector<PoissonHierarchyHost>&& probs, const SolverOp
     std::memset(const_cast<HostMailbox*>(mailbox_), 0, sizeof(HostMailbox));
     if (check(hipHostGetDevicePointer(reinterpret_cast<void**>(&mailbox_dev_), mailbox_, 0), "mailbox alias"))
         return -3;
-    if (block_max_leaves_ > 0 && check(block_kernels_init(), "block kernel attributes")) return -3;
     st_host_.assign(size_t(K), BatchPcg{});
     // level-to-kernel mapping: the faster of block-visit and per-sweep launches
     // for each merged coarse level (PoissonDevice::tune_levels), unless

@@ -2,10 +2,9 @@
 //
 // On the small levels of the hierarchy every smoothing sweep is its own
 // latency-bound launch. A block-visit kernel gives each leaf one workgroup
-// that stages the leaf plus a halo of H voxels (from up to 26 neighbour
-// leaves) in LDS and runs consecutive sweeps on a shrinking region: sweep k
-// is valid on [k, S-k)^3 of the S = 8 + 2H region, so after H-1 sweeps plus
-// the residual (or H sweeps) the leaf's own 8^3 values are exact. The halo
+// that holds the leaf plus a halo of 4 voxels (from up to 26 neighbour
+// leaves) and runs consecutive sweeps on a shrinking region: sweep k is valid
+// k voxels further in, so the leaf's own 8^3 values come out exact. The halo
 // voxels are recomputed redundantly by each neighbouring workgroup; every
 // value is produced by the same arithmetic as the per-sweep kernels
 // (stencil order ((x+ + x-) + (y+ + y-)) + (z+ + z-), fma(x, diag, s),
@@ -13,10 +12,19 @@
 // sweep's output is rounded where the per-sweep kernels store it, so results
 // are bit-identical to theirs in either precision.
 //
-//   kPreZero  (H = 3): x1 = w0 D^-1 b, two sweeps, residual, restriction
-//             (first visit, muCyclePreconditioner from a zero guess)
-//   kPreAgain (H = 4): three sweeps from the level's x, residual, restriction
-//   kPost     (H = 3): x + P x_coarse, three sweeps
+//   kPreZero   x1 = w0 D^-1 b, two sweeps, residual, restriction
+//              (first visit, muCyclePreconditioner from a zero guess)
+//   kPreAgain  three sweeps from the level's x, residual, restriction
+//   kPost      x + P x_coarse, three sweeps
+//
+// The region is 16^3 voxels, four of them in z per thread (1024 threads, one
+// wavefront per x slab): every global load is an aligned row of four values,
+// and each thread keeps its voxels' right-hand side and coefficients in
+// registers for all sweeps. Only x crosses threads, between slabs and y rows
+// through LDS (two buffers in turn, one barrier per sweep) and along z inside
+// the quad of lanes that holds a row. What bounds the kernel is latency: the
+// launch, two memory round trips (neighbourhood records, then operands) and
+// the chain of sweeps.
 //
 // On the level above the coarsest, the post-visit can take the coarsest solve
 // in with it (block_post_cg_kernel): every workgroup runs the coarsest CG on
@@ -36,21 +44,28 @@ namespace {
 using namespace dev;
 
 enum BlockMode { kPreZero = 0, kPreAgain = 1, kPost = 2 };
-constexpr int kBlkThreads = 512;
+constexpr int kBlkThreads = 1024;
 
-// LDS per region voxel: b, x, diag, invdiag, three face coefficients and the
-// mask byte (29 bytes; sweeps update x in place through registers), so two
-// H = 3 workgroups fit one CU's 160 KiB.
-template <int H>
-struct Region {
-    static constexpr int S = 8 + 2 * H;
-    static constexpr int N = S * S * S;
-    static constexpr size_t lds_bytes = size_t(N) * (7 * sizeof(float) + 1);
-};
-
-template <int H>
-__device__ __forceinline__ int ridx(int x, int y, int z) {
-    return (x * Region<H>::S + y) * Region<H>::S + z;
+// Loads of four values in z: a z row of four of a brick
+template <class V>
+__device__ __forceinline__ void ldq(const V* p, float v[4]) {
+    const float4 a = ld4(p);
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+}
+__device__ __forceinline__ void stq(float* p, const float v[4]) {
+    *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
+}
+__device__ __forceinline__ void stq(bf16* p, const float v[4]) {
+    *reinterpret_cast<uint2*>(p) = make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
+}
+__device__ __forceinline__ void ld2c(const float* p, float v[2]) {
+    const float2 a = *reinterpret_cast<const float2*>(p);
+    v[0] = a.x; v[1] = a.y;
+}
+__device__ __forceinline__ void ld2c(const bf16* p, float v[2]) {
+    const uint32_t q = *reinterpret_cast<const uint32_t*>(p);
+    v[0] = __uint_as_float(q << 16);
+    v[1] = __uint_as_float(q & 0xffff0000u);
 }
 
 // value as the vector storage type holds it (the per-sweep kernels store
@@ -61,209 +76,221 @@ __device__ __forceinline__ float stored(float v) {
     else return float(V(v));
 }
 
-// One Jacobi sweep x <- J_w(x) on [LO, S - LO)^3 of the region, each output
-// rounded to the storage type V: every thread computes its voxels into
-// registers, then, after a barrier, stores them (the caller's barrier
-// publishes the stores).
-template <int H, int LO, class V>
-__device__ __forceinline__ void sweep(float* x, const float* b, const float* dg, const float* inv, const float* cx,
-                                      const float* cy, const float* cz, const uint8_t* m, float w) {
-    constexpr int S = Region<H>::S;
-    constexpr int e = S - 2 * LO;
-    constexpr int cnt = e * e * e;
-    constexpr int kPer = (cnt + kBlkThreads - 1) / kBlkThreads;
-    float out[kPer];
-    int at[kPer];
+// v of the previous / next lane of the quad (a z row's four threads); the
+// quad's first / last lane gets its own value, which only voxels outside the
+// valid region use
+__device__ __forceinline__ float quad_prev(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x90, 0xf, 0xf, true));   // [0,0,1,2]
+}
+__device__ __forceinline__ float quad_next(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xf9, 0xf, 0xf, true));   // [1,2,3,3]
+}
+
+// A thread's four voxels: their right-hand side, coefficients and DOF bits.
+struct Quad {
+    float b[4], dg[4], inv[4], cx[4], cxp[4], cy[4], cyp[4], cz[4];
+    float czp;
+    uint32_t m;
+};
+
+// A x of the thread's voxels, x being its own values and `buf` the region's
+// (buf holds x of every thread; the caller has passed the barrier).
+__device__ __forceinline__ void quad_ax(const Quad& Q, const float4* buf, const float x[4], float ax[4]) {
+    const int t = threadIdx.x;
+    float s[4];
+    {
+        const float4 p = buf[t + 64], m = buf[t - 64];
+        const float xp[4] = {p.x, p.y, p.z, p.w}, xm[4] = {m.x, m.y, m.z, m.w};
 #pragma unroll
-    for (int k = 0; k < kPer; ++k) {
-        const int q = threadIdx.x + k * kBlkThreads;
-        at[k] = -1;
-        out[k] = 0.f;
-        if (q < cnt) {
-            const int vx = LO + q / (e * e), vy = LO + (q / e) % e, vz = LO + q % e;
-            const int i = ridx<H>(vx, vy, vz);
-            at[k] = i;
-            float r = 0.f;
-            if (m[i]) {
-                const int ix = S * S, iy = S;
-                const float f1 = x[i + ix] * cx[i + ix];
-                const float f2 = x[i - ix] * cx[i];
-                const float f3 = x[i + iy] * cy[i + iy];
-                const float f4 = x[i - iy] * cy[i];
-                const float f5 = x[i + 1] * cz[i + 1];
-                const float f6 = x[i - 1] * cz[i];
-                const float s = ((f1 + f2) + (f3 + f4)) + (f5 + f6);
-                const float ax = fmaf(x[i], dg[i], s);
-                float t = b[i] - ax;
-                t = t * inv[i];
-                r = fmaf(w, t, x[i]);
-            }
-            out[k] = stored<V>(r);
+        for (int k = 0; k < 4; ++k) {
+            const float f1 = xp[k] * Q.cxp[k];
+            const float f2 = xm[k] * Q.cx[k];
+            s[k] = f1 + f2;
         }
     }
-    __syncthreads();
+    {
+        const float4 p = buf[t + 4], m = buf[t - 4];
+        const float yp[4] = {p.x, p.y, p.z, p.w}, ym[4] = {m.x, m.y, m.z, m.w};
 #pragma unroll
-    for (int k = 0; k < kPer; ++k)
-        if (at[k] >= 0) x[at[k]] = out[k];
+        for (int k = 0; k < 4; ++k) {
+            const float f3 = yp[k] * Q.cyp[k];
+            const float f4 = ym[k] * Q.cy[k];
+            s[k] = s[k] + (f3 + f4);
+        }
+    }
+    const float zm = quad_prev(x[3]), zp = quad_next(x[0]);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const float f5 = (k < 3 ? x[k + 1] : zp) * (k < 3 ? Q.cz[k + 1] : Q.czp);
+        const float f6 = (k > 0 ? x[k - 1] : zm) * Q.cz[k];
+        s[k] = s[k] + (f5 + f6);
+        ax[k] = fmaf(x[k], Q.dg[k], s[k]);
+    }
+}
+
+// One Jacobi sweep x <- J_w(x), rounded to the storage type V, on slabs LO ..
+// 15 - LO (uniform per wavefront; rows outside LO .. 15 - LO in y, and the
+// outer z voxels, get values that nothing valid reads). x enters published in
+// `from`; it is published again in `to`.
+template <int LO, class V>
+__device__ __forceinline__ void sweep(const Quad& Q, const float4* from, float4* to, float x[4], float w) {
+    const int slab = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+    if (slab >= LO && slab <= 15 - LO) {
+        float ax[4];
+        quad_ax(Q, from, x, ax);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            float t = Q.b[k] - ax[k];
+            t = t * Q.inv[k];
+            const float r = fmaf(w, t, x[k]);
+            x[k] = ((Q.m >> k) & 1u) ? stored<V>(r) : 0.f;
+        }
+        to[threadIdx.x] = make_float4(x[0], x[1], x[2], x[3]);
+    }
+    __syncthreads();
 }
 
 // The visit of one leaf. kCg (kPost only): the coarse correction comes from
 // cgx, the coarsest solution in LDS indexed by coarsest DOF (dof_of maps a
 // coarsest brick position to its DOF, -1 elsewhere), instead of Xc.
-template <int H, int MODE, class V, bool kCg>
+template <int MODE, class V, bool kCg>
 __device__ __forceinline__ void visit_body(const LevelView& L, const V* Xin, const V* Xc, const V* B, V* Xout, V* Cv,
                                            float w0, float w1, float w2, const int32_t* dof_of, const float* cgx) {
-    constexpr int S = Region<H>::S, N = Region<H>::N;
-    extern __shared__ float lds[];
-    float* b = lds;
-    float* xa = b + N;
-    float* dg = xa + N;
-    float* inv = dg + N;
-    float* cx = inv + N;
-    float* cy = cx + N;
-    float* cz = cy + N;
-    uint8_t* m = reinterpret_cast<uint8_t*>(cz + N);
-    __shared__ int nl[27], sd[27], sx[27], sy[27], sz[27], par[27];
-
+    __shared__ float4 buf[2][kBlkThreads];
+    // the first region row the mode reads, and the first it sweeps
+    constexpr int kIn = MODE == kPreAgain ? 0 : 1;
+    constexpr int kSw = kIn + 1;
     const int leaf = logical_block();
     const int tid = threadIdx.x;
-    if (tid < 27) {
-        const int4* r = reinterpret_cast<const int4*>(L.nb27 + (size_t(leaf) * 27 + tid) * kNb27Stride);
-        const int4 a = r[0], b = r[1];
-        nl[tid] = a.x;
-        sd[tid] = a.y;
-        sx[tid] = a.z;
-        sy[tid] = a.w;
-        sz[tid] = b.x;
-        par[tid] = MODE == kPost ? b.y : -1;
-    }
-    __syncthreads();
+    const int slab = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ry = (tid >> 2) & 15, qz = tid & 3;
 
-    // stage the region: values of absent leaves are 0 (vectors, mask) or the
-    // default stencil constants (coefficients), as the per-sweep kernels read them
-    // unrolled so that every thread's loads are in flight together (the
-    // region's voxels are independent; one memory latency instead of one per
-    // pass of the loop)
-    constexpr int kPasses = (N + kBlkThreads - 1) / kBlkThreads;
+    // the record of the neighbourhood leaf that holds the thread's voxels
+    const int ax = slab < 4 ? 0 : (slab > 11 ? 2 : 1), ay = ry < 4 ? 0 : (ry > 11 ? 2 : 1);
+    const int az = qz < 1 ? 0 : (qz > 2 ? 2 : 1);
+    const int lx = (slab + 4) & 7, ly = (ry + 4) & 7, lz = 4 * ((qz + 1) & 1);
+    const int k27 = ax * 9 + ay * 3 + az;
+    const int32_t* rec = L.nb27 + (size_t(leaf) * 27 + k27) * kNb27Stride;
+    const int4 ra = *reinterpret_cast<const int4*>(rec);
+    const int2 rb = *reinterpret_cast<const int2*>(rec + 4);
+    // slots of the rows at x + 1 and y + 1 (the next neighbourhood leaf's past a face)
+    const int sxp = rec[(lx == 7 && ax < 2 ? 9 * kNb27Stride : 0) + 2];
+    const int syp = rec[(ly == 7 && ay < 2 ? 3 * kNb27Stride : 0) + 3];
+    const int n = ra.x;
+    const bool has = n >= 0;
+    const int row = (lx << 6) | (ly << 3) | lz;
+
+    Quad Q;
+    float x[4];
+    Q.m = 0;
 #pragma unroll
-    for (int pass = 0; pass < kPasses; ++pass) {
-        const int q = tid + pass * kBlkThreads;
-        if (q >= N) break;
-        const int gx = q / (S * S) - H, gy = (q / S) % S - H, gz = q % S - H;
-        const int ax = gx < 0 ? 0 : (gx > 7 ? 2 : 1), ay = gy < 0 ? 0 : (gy > 7 ? 2 : 1);
-        const int az = gz < 0 ? 0 : (gz > 7 ? 2 : 1);
-        const int k = ax * 9 + ay * 3 + az;
-        const int n = nl[k];
-        const int lx = gx & 7, ly = gy & 7, lz = gz & 7;
-        const int off = (lx << 6) | (ly << 3) | lz;
-        // every load is unconditional (absent leaf or slot: leaf 0 / slot 0,
-        // both exist, and the value is replaced below), so the loads of all
-        // passes are in flight together
-        const size_t nv = size_t(n >= 0 ? n : 0);
-        const int s0 = sd[k], s1 = sx[k], s2 = sy[k], s3 = sz[k];
-        const float tdg = L.diag[size_t(s0 >= 0 ? s0 : 0) * 512 + off];
-        const float tinv = L.invdiag[size_t(s0 >= 0 ? s0 : 0) * 512 + off];
-        const float tcx = L.cx[size_t(s1 >= 0 ? s1 : 0) * 512 + off];
-        const float tcy = L.cy[size_t(s2 >= 0 ? s2 : 0) * 512 + off];
-        const float tcz = L.cz[size_t(s3 >= 0 ? s3 : 0) * 512 + off];
-        uint64_t tm = L.mask[nv * 8 + lx];
-        float tb = float(B[nv * 512 + off]);
-        float tx = 0.f, tc = 0.f;
-        int pp = -1, di = -1;
-        if (MODE != kPreZero) tx = float(Xin[nv * 512 + off]);
-        if (MODE == kPost) {
-            pp = par[k];
-            const int p = pp >= 0 ? pp : 0, cl = p >> 3, oct = p & 7;
-            const int crow = ((lx >> 1) + 4 * ((oct >> 2) & 1)) * 8 + ((ly >> 1) + 4 * ((oct >> 1) & 1));
-            const size_t ci = size_t(cl) * 512 + crow * 8 + 4 * (oct & 1) + (lz >> 1);
-            if constexpr (kCg) di = dof_of[ci];
-            else tc = float(Xc[ci]);
-        }
-        // selects, no branches: the empty asm statements (no instruction)
-        // keep the compiler from sinking these loads into a branch on n
-        asm volatile("" : "+v"(tm), "+v"(tb), "+v"(tx), "+v"(tc), "+v"(di));
-        // a fine DOF's parent voxel is a coarsest DOF, the only case where tc is used
-        if constexpr (kCg) tc = cgx[di >= 0 ? di : kMaxCoarsestDof];
-        const bool has = n >= 0;
-        const float vdg = s0 >= 0 ? tdg : L.dflt_diag;
-        const float vinv = s0 >= 0 ? tinv : L.dflt_invdiag;
-        const uint8_t vm = has ? uint8_t((tm >> ((ly << 3) | lz)) & 1u) : uint8_t(0);
-        const float vb = has ? tb : 0.f;
-        float vx;
-        if (MODE == kPreZero) {
-            const float t = w0 * (vinv * vb);
-            vx = has ? t : 0.f;
-        } else {
-            vx = has ? tx : 0.f;
-            if (MODE == kPost) {
-                const float t = vx + tc;
-                vx = (vm && pp >= 0) ? t : vx;
+    for (int k = 0; k < 4; ++k) {
+        x[k] = 0.f;
+        Q.b[k] = 0.f;
+        Q.dg[k] = L.dflt_diag;
+        Q.inv[k] = L.dflt_invdiag;
+        Q.cx[k] = Q.cxp[k] = Q.cy[k] = Q.cyp[k] = Q.cz[k] = L.dflt_off;
+    }
+    if (slab >= kIn && slab <= 15 - kIn) {
+        // vectors of absent leaves are 0, coefficients of absent leaves or
+        // trimmed bricks the default constants
+        uint32_t mb = 0;
+        float c2[2] = {0.f, 0.f};
+        int di0 = -1, di1 = -1;
+        if (has) {
+            const size_t at = size_t(n) * 512 + row;
+            mb = reinterpret_cast<const uint8_t*>(L.mask)[size_t(n) * 64 + lx * 8 + ly];
+            ldq(B + at, Q.b);
+            if (MODE != kPreZero) ldq(Xin + at, x);
+            if (MODE == kPost && rb.y >= 0) {
+                const int cl = rb.y >> 3, oct = rb.y & 7;
+                const int crow = ((lx >> 1) + 4 * ((oct >> 2) & 1)) * 8 + ((ly >> 1) + 4 * ((oct >> 1) & 1));
+                const size_t ci = size_t(cl) * 512 + crow * 8 + 4 * (oct & 1) + (lz >> 1);
+                if constexpr (kCg) {
+                    const int2 d = *reinterpret_cast<const int2*>(dof_of + ci);
+                    di0 = d.x;
+                    di1 = d.y;
+                } else {
+                    ld2c(Xc + ci, c2);
+                }
             }
         }
-        b[q] = vb;
-        xa[q] = vx;
-        m[q] = vm;
-        dg[q] = vdg;
-        inv[q] = vinv;
-        cx[q] = s1 >= 0 ? tcx : L.dflt_off;
-        cy[q] = s2 >= 0 ? tcy : L.dflt_off;
-        cz[q] = s3 >= 0 ? tcz : L.dflt_off;
+        if (ra.y >= 0) {
+            ldq(L.diag + size_t(ra.y) * 512 + row, Q.dg);
+            ldq(L.invdiag + size_t(ra.y) * 512 + row, Q.inv);
+        }
+        if (slab >= kSw && slab <= 15 - kSw) {
+            if (ra.z >= 0) ldq(L.cx + size_t(ra.z) * 512 + row, Q.cx);
+            if (sxp >= 0) ldq(L.cx + size_t(sxp) * 512 + ((row + 64) & 511), Q.cxp);
+            if (ra.w >= 0) ldq(L.cy + size_t(ra.w) * 512 + row, Q.cy);
+            if (syp >= 0) ldq(L.cy + size_t(syp) * 512 + ((row & ~56) | ((row + 8) & 56)), Q.cyp);
+            if (rb.x >= 0) ldq(L.cz + size_t(rb.x) * 512 + row, Q.cz);
+        }
+        Q.m = (mb >> lz) & 15u;
+        if (MODE == kPreZero) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) x[k] = w0 * (Q.inv[k] * Q.b[k]);
+        }
+        if (MODE == kPost) {
+            if constexpr (kCg) {
+                // a fine DOF's parent voxel is a coarsest DOF, the only case where it is used
+                c2[0] = cgx[di0 >= 0 ? di0 : kMaxCoarsestDof];
+                c2[1] = cgx[di1 >= 0 ? di1 : kMaxCoarsestDof];
+            }
+            if (rb.y >= 0) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const float t = x[k] + c2[k >> 1];
+                    x[k] = ((Q.m >> k) & 1u) ? t : x[k];
+                }
+            }
+        }
     }
+    Q.czp = quad_next(Q.cz[0]);
+    buf[0][tid] = make_float4(x[0], x[1], x[2], x[3]);
     __syncthreads();
 
     if (MODE == kPreZero) {
-        sweep<H, 1, V>(xa, b, dg, inv, cx, cy, cz, m, w1);
-        __syncthreads();
-        sweep<H, 2, V>(xa, b, dg, inv, cx, cy, cz, m, w2);
-        __syncthreads();
+        sweep<2, V>(Q, buf[0], buf[1], x, w1);
+        sweep<3, V>(Q, buf[1], buf[0], x, w2);
+    } else if (MODE == kPreAgain) {
+        sweep<1, V>(Q, buf[0], buf[1], x, w0);
+        sweep<2, V>(Q, buf[1], buf[0], x, w1);
+        sweep<3, V>(Q, buf[0], buf[1], x, w2);
     } else {
-        sweep<H, 1, V>(xa, b, dg, inv, cx, cy, cz, m, w0);
-        __syncthreads();
-        sweep<H, 2, V>(xa, b, dg, inv, cx, cy, cz, m, w1);
-        __syncthreads();
-        sweep<H, 3, V>(xa, b, dg, inv, cx, cy, cz, m, w2);
-        __syncthreads();
+        sweep<2, V>(Q, buf[0], buf[1], x, w0);
+        sweep<3, V>(Q, buf[1], buf[0], x, w1);
+        sweep<4, V>(Q, buf[0], buf[1], x, w2);
     }
-    const float* fin = xa;   // the final sweep
 
-    // the leaf's own values
-    for (int q = tid; q < 512; q += kBlkThreads) {
-        const int i = ridx<H>(H + (q >> 6), H + ((q >> 3) & 7), H + (q & 7));
-        Xout[size_t(leaf) * 512 + q] = V(fin[i]);
-    }
+    // the leaf's own values: slabs and rows 4 .. 11, the two middle quads
+    const bool own = slab >= 4 && slab < 12 && ry >= 4 && ry < 12 && (qz == 1 || qz == 2);
+    if (own) stq(Xout + size_t(leaf) * 512 + row, x);
     if (MODE == kPost) return;
 
-    // residual on the own brick (into registers; then the first 512 entries
-    // of the diagonal array, no longer read, hold it), then restriction into
-    // the parent's octant
-    static_assert(kBlkThreads == 512, "one own-brick voxel per thread");
-    float rv = 0.f;
-    {
-        const int q = tid;
-        const int i = ridx<H>(H + (q >> 6), H + ((q >> 3) & 7), H + (q & 7));
-        if (m[i]) {
-            const int ix = S * S, iy = S;
-            const float* x = fin;
-            const float f1 = x[i + ix] * cx[i + ix];
-            const float f2 = x[i - ix] * cx[i];
-            const float f3 = x[i + iy] * cy[i + iy];
-            const float f4 = x[i - iy] * cy[i];
-            const float f5 = x[i + 1] * cz[i + 1];
-            const float f6 = x[i - 1] * cz[i];
-            const float s = ((f1 + f2) + (f3 + f4)) + (f5 + f6);
-            rv = b[i] - fmaf(x[i], dg[i], s);
-        }
+    // residual on the own brick, then restriction into the parent's octant;
+    // the buffer that the last sweep read holds the residual
+    const float4* fin = MODE == kPreZero ? buf[0] : buf[1];
+    float* rs = reinterpret_cast<float*>(MODE == kPreZero ? buf[1] : buf[0]);
+    if (slab >= 4 && slab < 12) {   // whole wavefronts: the quad exchange needs all four lanes
+        float axv[4], rv[4];
+        quad_ax(Q, fin, x, axv);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) rv[k] = ((Q.m >> k) & 1u) ? Q.b[k] - axv[k] : 0.f;
+        if (own) stq(rs + row, rv);
     }
-    __syncthreads();
-    float* rs = dg;
-    rs[tid] = rv;
     __syncthreads();
     if (tid < 64) {
         const int ccx = tid >> 4, ccy = (tid >> 2) & 3, ccz = tid & 3;
         float sum = 0.f;
+#pragma unroll
         for (int ii = 0; ii < 2; ++ii)
-            for (int jj = 0; jj < 2; ++jj)
-                for (int kk = 0; kk < 2; ++kk) sum += rs[((2 * ccx + ii) * 8 + (2 * ccy + jj)) * 8 + 2 * ccz + kk];
+#pragma unroll
+            for (int jj = 0; jj < 2; ++jj) {
+                const float2 r = *reinterpret_cast<const float2*>(rs + ((2 * ccx + ii) * 8 + (2 * ccy + jj)) * 8 + 2 * ccz);
+                sum += r.x;
+                sum += r.y;
+            }
         const int p = L.parent[leaf];
         if (p < 0) return;
         const int cl = p >> 3, oct = p & 7;
@@ -272,51 +299,33 @@ __device__ __forceinline__ void visit_body(const LevelView& L, const V* Xin, con
     }
 }
 
-template <int H, int MODE, class V>
-__global__ __launch_bounds__(kBlkThreads) void block_visit_kernel(LevelView L, const V* Xin, const V* Xc, const V* B,
-                                                                  V* Xout, V* Cv, float w0, float w1, float w2) {
-    visit_body<H, MODE, V, false>(L, Xin, Xc, B, Xout, Cv, w0, w1, w2, nullptr, nullptr);
+template <int MODE, class V>
+__global__ __launch_bounds__(kBlkThreads) __attribute__((amdgpu_waves_per_eu(8))) void block_visit_kernel(
+    LevelView L, const V* Xin, const V* Xc, const V* B, V* Xout, V* Cv, float w0, float w1, float w2) {
+    visit_body<MODE, V, false>(L, Xin, Xc, B, Xout, Cv, w0, w1, w2, nullptr, nullptr);
 }
 
 // The coarsest solve (right-hand side Bc, solution stored into Xc by
 // workgroup 0) followed by the kPost visit of the level above it. The CG's
-// last barrier has passed when it writes its solution into cg.sp, and the
-// visit's first barrier publishes it.
+// last barrier has passed when it writes its solution into cg.sp; the barrier
+// here publishes it.
 template <class V, int kMaxDof>
 __global__ __launch_bounds__(kBlkThreads) void block_post_cg_kernel(LevelView L, CoarsestView C,
                                                                     const int32_t* dof_of, const V* Bc, V* Xc,
                                                                     const V* Xin, const V* B, V* Xout, float w0,
                                                                     float w1, float w2) {
+    static_assert(kBlkThreads == kCgThreads, "the standalone solve's thread count");
     __shared__ CgShared<kBlkThreads> cg;
     coarsest_cg_block<kBlkThreads, V, kMaxDof, true>(C, Bc, blockIdx.x == 0 ? Xc : nullptr, cg);
-    visit_body<3, kPost, V, true>(L, Xin, nullptr, B, Xout, nullptr, w0, w1, w2, dof_of, cg.sp);
+    __syncthreads();
+    visit_body<kPost, V, true>(L, Xin, nullptr, B, Xout, nullptr, w0, w1, w2, dof_of, cg.sp);
 }
 
-template <int H, int MODE, class V>
+template <int MODE, class V>
 hipError_t launch_mode(const LevelView& L, const V* xin, const V* xc, const V* b, V* xout, V* cv, float w0, float w1,
                        float w2, hipStream_t s) {
-    block_visit_kernel<H, MODE, V><<<unsigned(L.nleaf), kBlkThreads, Region<H>::lds_bytes, s>>>(L, xin, xc, b, xout,
-                                                                                                cv, w0, w1, w2);
+    block_visit_kernel<MODE, V><<<unsigned(L.nleaf), kBlkThreads, 0, s>>>(L, xin, xc, b, xout, cv, w0, w1, w2);
     return hipGetLastError();
-}
-
-template <class V>
-hipError_t set_lds_limits() {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&block_visit_kernel<3, kPreZero, V>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, int(Region<3>::lds_bytes));
-    if (e == hipSuccess)
-        e = hipFuncSetAttribute(reinterpret_cast<const void*>(&block_visit_kernel<4, kPreAgain, V>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, int(Region<4>::lds_bytes));
-    if (e == hipSuccess)
-        e = hipFuncSetAttribute(reinterpret_cast<const void*>(&block_visit_kernel<3, kPost, V>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, int(Region<3>::lds_bytes));
-    if (e == hipSuccess)
-        e = hipFuncSetAttribute(reinterpret_cast<const void*>(&block_post_cg_kernel<V, kCgSmallDof>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, int(Region<3>::lds_bytes));
-    if (e == hipSuccess)
-        e = hipFuncSetAttribute(reinterpret_cast<const void*>(&block_post_cg_kernel<V, kMaxCoarsestDof>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, int(Region<3>::lds_bytes));
-    return e;
 }
 
 template <class V>
@@ -324,8 +333,8 @@ hipError_t block_pre_t(const LevelView& L, bool from_zero, const V* x, const V* 
                        float w1, float w2, hipStream_t s) {
     if (L.nleaf <= 0) return hipSuccess;
     if (!L.nb27) return hipErrorInvalidValue;
-    if (from_zero) return launch_mode<3, kPreZero, V>(L, nullptr, nullptr, b, x_out, coarse_b, w0, w1, w2, s);
-    return launch_mode<4, kPreAgain, V>(L, x, nullptr, b, x_out, coarse_b, w0, w1, w2, s);
+    if (from_zero) return launch_mode<kPreZero, V>(L, nullptr, nullptr, b, x_out, coarse_b, w0, w1, w2, s);
+    return launch_mode<kPreAgain, V>(L, x, nullptr, b, x_out, coarse_b, w0, w1, w2, s);
 }
 
 template <class V>
@@ -333,7 +342,7 @@ hipError_t block_post_t(const LevelView& L, const V* x, const V* xc, const V* b,
                         hipStream_t s) {
     if (L.nleaf <= 0) return hipSuccess;
     if (!L.nb27) return hipErrorInvalidValue;
-    return launch_mode<3, kPost, V>(L, x, xc, b, x_out, nullptr, w0, w1, w2, s);
+    return launch_mode<kPost, V>(L, x, xc, b, x_out, nullptr, w0, w1, w2, s);
 }
 
 template <class V>
@@ -342,22 +351,15 @@ hipError_t block_post_cg_t(const LevelView& L, const CoarsestView& C, const int3
     if (L.nleaf <= 0) return hipSuccess;   // as block_post_t: nothing reads the coarse correction
     if (!L.nb27 || !dof_of || C.ndof <= 0 || C.ndof > kMaxCoarsestDof) return hipErrorInvalidValue;
     const unsigned g = unsigned(L.nleaf);
-    const size_t lds = Region<3>::lds_bytes;
     if (C.ndof <= kCgSmallDof)
-        block_post_cg_kernel<V, kCgSmallDof><<<g, kBlkThreads, lds, s>>>(L, C, dof_of, bc, xc, x, b, x_out, w0, w1, w2);
+        block_post_cg_kernel<V, kCgSmallDof><<<g, kBlkThreads, 0, s>>>(L, C, dof_of, bc, xc, x, b, x_out, w0, w1, w2);
     else
         block_post_cg_kernel<V, kMaxCoarsestDof>
-            <<<g, kBlkThreads, lds, s>>>(L, C, dof_of, bc, xc, x, b, x_out, w0, w1, w2);
+            <<<g, kBlkThreads, 0, s>>>(L, C, dof_of, bc, xc, x, b, x_out, w0, w1, w2);
     return hipGetLastError();
 }
 
 }  // namespace
-
-hipError_t block_kernels_init() {
-    hipError_t e = set_lds_limits<float>();
-    if (e == hipSuccess) e = set_lds_limits<bf16>();
-    return e;
-}
 
 hipError_t launch_block_pre(const LevelView& L, bool from_zero, const float* x, const float* b, float* x_out,
                             float* coarse_b, float w0, float w1, float w2, hipStream_t s) {

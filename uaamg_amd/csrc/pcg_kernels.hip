@@ -351,14 +351,14 @@ __global__ __launch_bounds__(kBlockThreads) void update_kernel(LevelView L, cons
 }
 
 // ---------------------------------------------------------- coarsest solve
-// Workgroup size of the coarsest CG: 512 threads by default; UAAMG_CG_THREADS = 256 or
-// 1024 selects another (a tuning knob: the reductions' partial sums then group
+// Workgroup size of the coarsest CG: kCgThreads by default; UAAMG_CG_THREADS = 256 or
+// 512 selects another (a tuning knob: the reductions' partial sums then group
 // differently, so single and batched solves must run with the same setting).
 int cg_threads() {
     static const int t = [] {
         const char* e = std::getenv("UAAMG_CG_THREADS");
-        const int v = e ? std::atoi(e) : 512;
-        return (v == 256 || v == 1024) ? v : 512;
+        const int v = e ? std::atoi(e) : kCgThreads;
+        return (v == 256 || v == 512) ? v : kCgThreads;
     }();
     return t;
 }
@@ -719,10 +719,10 @@ hipError_t launch_cg_variant(bool batched, const CoarsestView* views, const Coar
     } while (0)
     if (small) {
         if (t == 256) UAAMG_CG_LAUNCH(kCgSmallDof, 256);
-        else if (t == 1024) UAAMG_CG_LAUNCH(kCgSmallDof, 1024);
-        else UAAMG_CG_LAUNCH(kCgSmallDof, 512);
+        else if (t == 512) UAAMG_CG_LAUNCH(kCgSmallDof, 512);
+        else UAAMG_CG_LAUNCH(kCgSmallDof, kCgThreads);
     } else {
-        if (t == 1024) UAAMG_CG_LAUNCH(kMaxCoarsestDof, 1024);
+        if (t == kCgThreads) UAAMG_CG_LAUNCH(kMaxCoarsestDof, kCgThreads);
         else UAAMG_CG_LAUNCH(kMaxCoarsestDof, 512);
     }
 #undef UAAMG_CG_LAUNCH

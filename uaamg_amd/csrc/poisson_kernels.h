@@ -167,8 +167,14 @@ struct TailArgs {
 constexpr int kWavesPerBlock = 4;
 constexpr int kBlockThreads = 64 * kWavesPerBlock;
 constexpr int kMaxCoarsestDof = 4096;
-// coarsest systems up to this size keep four row slots per thread of a
-// 512-thread solve (fewer registers; about 8% faster at ~1700 DOF)
+// Workgroup size of the coarsest CG. The grouping of its sums depends on it, so
+// every kernel that solves the coarsest system (standalone, batched, inside a
+// block post-visit, in the tail kernel) uses the same. A full-size workgroup
+// keeps two rows per thread at 2048 rows, where the serial work per thread is
+// what an iteration waits for.
+constexpr int kCgThreads = 1024;
+// coarsest systems up to this size keep two row slots per thread (fewer
+// registers and less serial work than the four of the full size)
 constexpr int kCgSmallDof = 2048;
 
 // ---- launchers (stream-ordered, no host synchronisation) ----
@@ -228,8 +234,7 @@ hipError_t launch_update_laplacian_dot(const LevelView& L, const float* z, const
 // x += alpha p only (final step)
 hipError_t launch_update_x(const LevelView& L, const float* p, float* x, const PcgScalars* sc, hipStream_t s);
 
-// ---- block-visit kernels (one workgroup per leaf, halo staged in LDS; needs L.nb27)
-hipError_t block_kernels_init();
+// ---- block-visit kernels (one workgroup per leaf and its halo; needs L.nb27)
 // pre-smoothing (3 weighted Jacobi sweeps w0, w1, w2; from a zero guess when
 // from_zero, else from x) into x_out, and coarse_b = R (b - A x_out)
 hipError_t launch_block_pre(const LevelView& L, bool from_zero, const float* x, const float* b, float* x_out,
@@ -240,14 +245,14 @@ hipError_t launch_block_post(const LevelView& L, const float* x, const float* xc
 // The coarsest solve xc = CG(bc) (as launch_coarsest_cg stores it) and then
 // launch_block_post of the level above the coarsest with that xc, in one
 // launch. dof_of: [coarsest leaves * 512], the coarsest DOF at each brick
-// position or -1. Requires the coarsest CG at 512 threads.
+// position or -1. Requires the coarsest CG at kCgThreads threads.
 hipError_t launch_block_post_cg(const LevelView& L, const CoarsestView& C, const int32_t* dof_of, const float* bc,
                                 float* xc, const float* x, const float* b, float* x_out, float w0, float w1, float w2,
                                 hipStream_t s);
 hipError_t launch_block_post_cg(const LevelView& L, const CoarsestView& C, const int32_t* dof_of, const bf16* bc,
                                 bf16* xc, const bf16* x, const bf16* b, bf16* x_out, float w0, float w1, float w2,
                                 hipStream_t s);
-// threads of the coarsest CG workgroup (512 unless UAAMG_CG_THREADS says otherwise)
+// threads of the coarsest CG workgroup (kCgThreads unless UAAMG_CG_THREADS says otherwise)
 int coarsest_cg_threads();
 
 // ---- mixed-precision W-cycle: the same passes with the level vectors stored

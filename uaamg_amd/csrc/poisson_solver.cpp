@@ -435,7 +435,6 @@ int PoissonDevice::acquire_device() {
         use_block_.assign(size_t(L), 0);
         for (int l = 1; l + 1 < L; ++l)
             use_block_[size_t(l)] = int64_t(host_.levels[l].nleaf()) <= block_max_leaves_ ? 1 : 0;
-        if (block_max_leaves_ > 0 && check(block_kernels_init(), "block kernel attributes")) return -3;
         tune_pending = block_max_leaves_ > 0 && !fixed;
     }
     if (opt_.precision != 0 && opt_.precision != 1) {
@@ -928,7 +927,7 @@ int PoissonDevice::build_coarsest() {
     for (int64_t d = 0; d < nd; ++d) dof_of[size_t(pos[size_t(d)])] = int32_t(d);
     coarsest_dof_of_ = static_cast<const int32_t*>(up(dof_of.data(), dof_of.size() * sizeof(int32_t)));
     const char* env = std::getenv("UAAMG_POST_CG");
-    post_cg_ = nd > 0 && coarsest_dof_of_ && coarsest_cg_threads() == 512 && !(env && env[0] == '0');
+    post_cg_ = nd > 0 && coarsest_dof_of_ && coarsest_cg_threads() == kCgThreads && !(env && env[0] == '0');
     if (check(hipStreamSynchronize(stream_), "coarsest upload")) return -3;
     return 0;
 }

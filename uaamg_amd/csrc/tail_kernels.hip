@@ -4,11 +4,11 @@
 // <= 4000 DOFs and the one above it roughly 8x that), so a separate launch per
 // sweep there costs more in launch latency than in work. The tail kernel runs
 // both mu = 2 visits of level L-2 (muCyclePreconditioner<2,...> called twice
-// from level L-3, simd_vdb_poisson.cpp:1932-1935) on one 512-thread workgroup:
+// from level L-3, simd_vdb_poisson.cpp:1932-1935) on one workgroup:
 // pre-smoothing, residual + restriction, the coarsest solve, prolongation fused
 // into the first post-smoothing sweep, two more sweeps — with a workgroup
-// barrier between phases (512 threads: the coarsest rows of 8 DOFs per
-// thread stay in registers). The arithmetic per value is exactly that of the
+// barrier between phases (the coarsest CG's thread count, so its rows stay in
+// registers and its sums group as in the standalone solve). The arithmetic per value is exactly that of the
 // per-sweep kernels (same device routines), only the launch structure changes.
 #include "coarsest_device.h"
 #include "stencil_device.h"
@@ -18,7 +18,7 @@ namespace {
 
 using namespace dev;
 
-constexpr int kTailThreads = 512;
+constexpr int kTailThreads = kCgThreads;
 constexpr int kTailWaves = kTailThreads / 64;
 
 struct TailShared {
