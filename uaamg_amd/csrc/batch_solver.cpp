@@ -200,12 +200,14 @@ int PoissonBatch::init(std::vector<PoissonHierarchyHost>&& probs, const SolverOp
         complete_leaf_records(H[size_t(l)].slot.data(), H[size_t(l)].nbr.data(), H[size_t(l)].parent.data(),
                               size_t(nleaf[size_t(l)]));
     // coarsest systems, merged order
-    std::vector<std::vector<int32_t>> cpos(static_cast<size_t>(K)), cnb(static_cast<size_t>(K));
+    std::vector<std::vector<int32_t>> crow(static_cast<size_t>(K));
     std::vector<std::vector<float>> ccoef(static_cast<size_t>(K));
     for (int k = 0; k < K; ++k) {
         const int c = nlev_[size_t(k)] - 1;
-        coarsest_system(hl(k, c), off[size_t(c)][size_t(k)], cpos[size_t(k)], cnb[size_t(k)], ccoef[size_t(k)]);
-        lv_[size_t(c)].coarse_max_ndof = std::max(lv_[size_t(c)].coarse_max_ndof, int(cpos[size_t(k)].size()));
+        std::vector<int32_t> pos, nb;
+        coarsest_system(hl(k, c), off[size_t(c)][size_t(k)], pos, nb, ccoef[size_t(k)]);
+        crow[size_t(k)] = coarsest_rows(pos, nb);
+        lv_[size_t(c)].coarse_max_ndof = std::max(lv_[size_t(c)].coarse_max_ndof, int(pos.size()));
     }
 
     // one arena for everything
@@ -228,7 +230,7 @@ int PoissonBatch::init(std::vector<PoissonHierarchyHost>&& probs, const SolverOp
     bytes += al((n0 / kWavesPerBlock + 16) * 8);              // partials
     bytes += al(size_t(K) * sizeof(BatchPcg)) + al(64) + al(size_t(K) * sizeof(CoarsestView));
     for (int k = 0; k < K; ++k)
-        bytes += al(cpos[size_t(k)].size() * 4) + al(cnb[size_t(k)].size() * 4) + al(ccoef[size_t(k)].size() * 4);
+        bytes += al(crow[size_t(k)].size() * 4) + al(ccoef[size_t(k)].size() * 4);
 
     if (check(hipSetDevice(opt_.device), "hipSetDevice")) return -3;
     if (opt_.stream) {
@@ -325,8 +327,7 @@ int PoissonBatch::init(std::vector<PoissonHierarchyHost>&& probs, const SolverOp
         for (int k = 0; k < K; ++k) {
             CoarsestView& cv = views[size_t(k)];
             cv.ndof = int32_t(hl(k, nlev_[size_t(k)] - 1).ndof);
-            cv.pos = static_cast<const int32_t*>(up(cpos[size_t(k)].data(), cpos[size_t(k)].size() * 4));
-            cv.nb = static_cast<const int32_t*>(up(cnb[size_t(k)].data(), cnb[size_t(k)].size() * 4));
+            cv.row = static_cast<const int32_t*>(up(crow[size_t(k)].data(), crow[size_t(k)].size() * 4));
             cv.coef = static_cast<const float*>(up(ccoef[size_t(k)].data(), ccoef[size_t(k)].size() * 4));
             cv.max_iters = 10;
             cv.tol = FLT_EPSILON;

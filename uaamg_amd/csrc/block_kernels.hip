@@ -44,6 +44,10 @@ namespace {
 using namespace dev;
 
 enum BlockMode { kPreZero = 0, kPreAgain = 1, kPost = 2 };
+constexpr int kRegionQuads = 1024;   // 16 x 16 rows of four quads
+// One quad per thread: with two per thread and half the threads the visit pair
+// of a 282-leaf level took 34.1 us against 32.5 (VALU time per sweep is the
+// same, fewer wavefronts hide less of the loads).
 constexpr int kBlkThreads = 1024;
 
 // Loads of four values in z: a z row of four of a brick
@@ -93,10 +97,9 @@ struct Quad {
     uint32_t m;
 };
 
-// A x of the thread's voxels, x being its own values and `buf` the region's
-// (buf holds x of every thread; the caller has passed the barrier).
-__device__ __forceinline__ void quad_ax(const Quad& Q, const float4* buf, const float x[4], float ax[4]) {
-    const int t = threadIdx.x;
+// A x of the quad at region index t, x being its own values and `buf` the
+// region's (buf holds x of every quad; the caller has passed the barrier).
+__device__ __forceinline__ void quad_ax(const Quad& Q, const float4* buf, int t, const float x[4], float ax[4]) {
     float s[4];
     {
         const float4 p = buf[t + 64], m = buf[t - 64];
@@ -128,24 +131,42 @@ __device__ __forceinline__ void quad_ax(const Quad& Q, const float4* buf, const 
     }
 }
 
+// A workgroup of kT threads: 1024 / kT quads per thread, wavefront w holding
+// slabs w, w + kT/64, ...
+template <int kT>
+struct Part {
+    static constexpr int kPer = kRegionQuads / kT;
+    Quad Q[kPer];
+    float x[kPer][4];
+    __device__ __forceinline__ static int slab(int h) {
+        return __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)) + h * (kT / 64);
+    }
+    __device__ __forceinline__ static int at(int h) { return int(threadIdx.x) + h * kT; }
+};
+
 // One Jacobi sweep x <- J_w(x), rounded to the storage type V, on slabs LO ..
 // 15 - LO (uniform per wavefront; rows outside LO .. 15 - LO in y, and the
 // outer z voxels, get values that nothing valid reads). x enters published in
 // `from`; it is published again in `to`.
-template <int LO, class V>
-__device__ __forceinline__ void sweep(const Quad& Q, const float4* from, float4* to, float x[4], float w) {
-    const int slab = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
-    if (slab >= LO && slab <= 15 - LO) {
-        float ax[4];
-        quad_ax(Q, from, x, ax);
+template <int LO, class V, int kT>
+__device__ __forceinline__ void sweep(Part<kT>& P, const float4* from, float4* to, float w) {
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            float t = Q.b[k] - ax[k];
-            t = t * Q.inv[k];
-            const float r = fmaf(w, t, x[k]);
-            x[k] = ((Q.m >> k) & 1u) ? stored<V>(r) : 0.f;
+    for (int h = 0; h < Part<kT>::kPer; ++h) {
+        const int slab = P.slab(h);
+        if (slab >= LO && slab <= 15 - LO) {
+            const Quad& Q = P.Q[h];
+            float* x = P.x[h];
+            float ax[4];
+            quad_ax(Q, from, P.at(h), x, ax);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                float t = Q.b[k] - ax[k];
+                t = t * Q.inv[k];
+                const float r = fmaf(w, t, x[k]);
+                x[k] = ((Q.m >> k) & 1u) ? stored<V>(r) : 0.f;
+            }
+            to[P.at(h)] = make_float4(x[0], x[1], x[2], x[3]);
         }
-        to[threadIdx.x] = make_float4(x[0], x[1], x[2], x[3]);
     }
     __syncthreads();
 }
@@ -153,132 +174,146 @@ __device__ __forceinline__ void sweep(const Quad& Q, const float4* from, float4*
 // The visit of one leaf. kCg (kPost only): the coarse correction comes from
 // cgx, the coarsest solution in LDS indexed by coarsest DOF (dof_of maps a
 // coarsest brick position to its DOF, -1 elsewhere), instead of Xc.
-template <int MODE, class V, bool kCg>
+template <int MODE, class V, int kT, bool kCg>
 __device__ __forceinline__ void visit_body(const LevelView& L, const V* Xin, const V* Xc, const V* B, V* Xout, V* Cv,
                                            float w0, float w1, float w2, const int32_t* dof_of, const float* cgx) {
-    __shared__ float4 buf[2][kBlkThreads];
+    __shared__ float4 buf[2][kRegionQuads];
     // the first region row the mode reads, and the first it sweeps
     constexpr int kIn = MODE == kPreAgain ? 0 : 1;
     constexpr int kSw = kIn + 1;
+    constexpr int kPer = Part<kT>::kPer;
+    Part<kT> P;
     const int leaf = logical_block();
     const int tid = threadIdx.x;
-    const int slab = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ry = (tid >> 2) & 15, qz = tid & 3;
+    const int ay = ry < 4 ? 0 : (ry > 11 ? 2 : 1), az = qz < 1 ? 0 : (qz > 2 ? 2 : 1);
+    const int ly = (ry + 4) & 7, lz = 4 * ((qz + 1) & 1);
 
-    // the record of the neighbourhood leaf that holds the thread's voxels
-    const int ax = slab < 4 ? 0 : (slab > 11 ? 2 : 1), ay = ry < 4 ? 0 : (ry > 11 ? 2 : 1);
-    const int az = qz < 1 ? 0 : (qz > 2 ? 2 : 1);
-    const int lx = (slab + 4) & 7, ly = (ry + 4) & 7, lz = 4 * ((qz + 1) & 1);
-    const int k27 = ax * 9 + ay * 3 + az;
-    const int32_t* rec = L.nb27 + (size_t(leaf) * 27 + k27) * kNb27Stride;
-    const int4 ra = *reinterpret_cast<const int4*>(rec);
-    const int2 rb = *reinterpret_cast<const int2*>(rec + 4);
-    // slots of the rows at x + 1 and y + 1 (the next neighbourhood leaf's past a face)
-    const int sxp = rec[(lx == 7 && ax < 2 ? 9 * kNb27Stride : 0) + 2];
-    const int syp = rec[(ly == 7 && ay < 2 ? 3 * kNb27Stride : 0) + 3];
-    const int n = ra.x;
-    const bool has = n >= 0;
-    const int row = (lx << 6) | (ly << 3) | lz;
-
-    Quad Q;
-    float x[4];
-    Q.m = 0;
+    // the records of the neighbourhood leaves that hold the thread's voxels
+    int4 ra[kPer];
+    int2 rb[kPer];
+    int sxp[kPer], syp[kPer];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        x[k] = 0.f;
-        Q.b[k] = 0.f;
-        Q.dg[k] = L.dflt_diag;
-        Q.inv[k] = L.dflt_invdiag;
-        Q.cx[k] = Q.cxp[k] = Q.cy[k] = Q.cyp[k] = Q.cz[k] = L.dflt_off;
+    for (int h = 0; h < kPer; ++h) {
+        const int slab = P.slab(h);
+        const int ax = slab < 4 ? 0 : (slab > 11 ? 2 : 1), lx = (slab + 4) & 7;
+        const int32_t* rec = L.nb27 + (size_t(leaf) * 27 + ax * 9 + ay * 3 + az) * kNb27Stride;
+        ra[h] = *reinterpret_cast<const int4*>(rec);
+        rb[h] = *reinterpret_cast<const int2*>(rec + 4);
+        // slots of the rows at x + 1 and y + 1 (the next neighbourhood leaf's past a face)
+        sxp[h] = rec[(lx == 7 && ax < 2 ? 9 * kNb27Stride : 0) + 2];
+        syp[h] = rec[(ly == 7 && ay < 2 ? 3 * kNb27Stride : 0) + 3];
     }
-    if (slab >= kIn && slab <= 15 - kIn) {
-        // vectors of absent leaves are 0, coefficients of absent leaves or
-        // trimmed bricks the default constants
-        uint32_t mb = 0;
-        float c2[2] = {0.f, 0.f};
-        int di0 = -1, di1 = -1;
-        if (has) {
-            const size_t at = size_t(n) * 512 + row;
-            mb = reinterpret_cast<const uint8_t*>(L.mask)[size_t(n) * 64 + lx * 8 + ly];
-            ldq(B + at, Q.b);
-            if (MODE != kPreZero) ldq(Xin + at, x);
-            if (MODE == kPost && rb.y >= 0) {
-                const int cl = rb.y >> 3, oct = rb.y & 7;
-                const int crow = ((lx >> 1) + 4 * ((oct >> 2) & 1)) * 8 + ((ly >> 1) + 4 * ((oct >> 1) & 1));
-                const size_t ci = size_t(cl) * 512 + crow * 8 + 4 * (oct & 1) + (lz >> 1);
+#pragma unroll
+    for (int h = 0; h < kPer; ++h) {
+        const int slab = P.slab(h);
+        const int lx = (slab + 4) & 7;
+        const int n = ra[h].x;
+        const int row = (lx << 6) | (ly << 3) | lz;
+        Quad& Q = P.Q[h];
+        float* x = P.x[h];
+        Q.m = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            x[k] = 0.f;
+            Q.b[k] = 0.f;
+            Q.dg[k] = L.dflt_diag;
+            Q.inv[k] = L.dflt_invdiag;
+            Q.cx[k] = Q.cxp[k] = Q.cy[k] = Q.cyp[k] = Q.cz[k] = L.dflt_off;
+        }
+        if (slab >= kIn && slab <= 15 - kIn) {
+            // vectors of absent leaves are 0, coefficients of absent leaves or
+            // trimmed bricks the default constants
+            uint32_t mb = 0;
+            float c2[2] = {0.f, 0.f};
+            int di0 = -1, di1 = -1;
+            if (n >= 0) {
+                const size_t at = size_t(n) * 512 + row;
+                mb = reinterpret_cast<const uint8_t*>(L.mask)[size_t(n) * 64 + lx * 8 + ly];
+                ldq(B + at, Q.b);
+                if (MODE != kPreZero) ldq(Xin + at, x);
+                if (MODE == kPost && rb[h].y >= 0) {
+                    const int cl = rb[h].y >> 3, oct = rb[h].y & 7;
+                    const int crow = ((lx >> 1) + 4 * ((oct >> 2) & 1)) * 8 + ((ly >> 1) + 4 * ((oct >> 1) & 1));
+                    const size_t ci = size_t(cl) * 512 + crow * 8 + 4 * (oct & 1) + (lz >> 1);
+                    if constexpr (kCg) {
+                        const int2 d = *reinterpret_cast<const int2*>(dof_of + ci);
+                        di0 = d.x;
+                        di1 = d.y;
+                    } else {
+                        ld2c(Xc + ci, c2);
+                    }
+                }
+            }
+            if (ra[h].y >= 0) {
+                ldq(L.diag + size_t(ra[h].y) * 512 + row, Q.dg);
+                ldq(L.invdiag + size_t(ra[h].y) * 512 + row, Q.inv);
+            }
+            if (slab >= kSw && slab <= 15 - kSw) {
+                if (ra[h].z >= 0) ldq(L.cx + size_t(ra[h].z) * 512 + row, Q.cx);
+                if (sxp[h] >= 0) ldq(L.cx + size_t(sxp[h]) * 512 + ((row + 64) & 511), Q.cxp);
+                if (ra[h].w >= 0) ldq(L.cy + size_t(ra[h].w) * 512 + row, Q.cy);
+                if (syp[h] >= 0) ldq(L.cy + size_t(syp[h]) * 512 + ((row & ~56) | ((row + 8) & 56)), Q.cyp);
+                if (rb[h].x >= 0) ldq(L.cz + size_t(rb[h].x) * 512 + row, Q.cz);
+            }
+            Q.m = (mb >> lz) & 15u;
+            if (MODE == kPreZero) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) x[k] = w0 * (Q.inv[k] * Q.b[k]);
+            }
+            if (MODE == kPost) {
                 if constexpr (kCg) {
-                    const int2 d = *reinterpret_cast<const int2*>(dof_of + ci);
-                    di0 = d.x;
-                    di1 = d.y;
-                } else {
-                    ld2c(Xc + ci, c2);
+                    // a fine DOF's parent voxel is a coarsest DOF, the only case where it is used
+                    c2[0] = cgx[di0 >= 0 ? di0 : kMaxCoarsestDof];
+                    c2[1] = cgx[di1 >= 0 ? di1 : kMaxCoarsestDof];
+                }
+                if (rb[h].y >= 0) {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const float t = x[k] + c2[k >> 1];
+                        x[k] = ((Q.m >> k) & 1u) ? t : x[k];
+                    }
                 }
             }
         }
-        if (ra.y >= 0) {
-            ldq(L.diag + size_t(ra.y) * 512 + row, Q.dg);
-            ldq(L.invdiag + size_t(ra.y) * 512 + row, Q.inv);
-        }
-        if (slab >= kSw && slab <= 15 - kSw) {
-            if (ra.z >= 0) ldq(L.cx + size_t(ra.z) * 512 + row, Q.cx);
-            if (sxp >= 0) ldq(L.cx + size_t(sxp) * 512 + ((row + 64) & 511), Q.cxp);
-            if (ra.w >= 0) ldq(L.cy + size_t(ra.w) * 512 + row, Q.cy);
-            if (syp >= 0) ldq(L.cy + size_t(syp) * 512 + ((row & ~56) | ((row + 8) & 56)), Q.cyp);
-            if (rb.x >= 0) ldq(L.cz + size_t(rb.x) * 512 + row, Q.cz);
-        }
-        Q.m = (mb >> lz) & 15u;
-        if (MODE == kPreZero) {
-#pragma unroll
-            for (int k = 0; k < 4; ++k) x[k] = w0 * (Q.inv[k] * Q.b[k]);
-        }
-        if (MODE == kPost) {
-            if constexpr (kCg) {
-                // a fine DOF's parent voxel is a coarsest DOF, the only case where it is used
-                c2[0] = cgx[di0 >= 0 ? di0 : kMaxCoarsestDof];
-                c2[1] = cgx[di1 >= 0 ? di1 : kMaxCoarsestDof];
-            }
-            if (rb.y >= 0) {
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const float t = x[k] + c2[k >> 1];
-                    x[k] = ((Q.m >> k) & 1u) ? t : x[k];
-                }
-            }
-        }
+        Q.czp = quad_next(Q.cz[0]);
+        buf[0][P.at(h)] = make_float4(x[0], x[1], x[2], x[3]);
     }
-    Q.czp = quad_next(Q.cz[0]);
-    buf[0][tid] = make_float4(x[0], x[1], x[2], x[3]);
     __syncthreads();
 
     if (MODE == kPreZero) {
-        sweep<2, V>(Q, buf[0], buf[1], x, w1);
-        sweep<3, V>(Q, buf[1], buf[0], x, w2);
+        sweep<2, V, kT>(P, buf[0], buf[1], w1);
+        sweep<3, V, kT>(P, buf[1], buf[0], w2);
     } else if (MODE == kPreAgain) {
-        sweep<1, V>(Q, buf[0], buf[1], x, w0);
-        sweep<2, V>(Q, buf[1], buf[0], x, w1);
-        sweep<3, V>(Q, buf[0], buf[1], x, w2);
+        sweep<1, V, kT>(P, buf[0], buf[1], w0);
+        sweep<2, V, kT>(P, buf[1], buf[0], w1);
+        sweep<3, V, kT>(P, buf[0], buf[1], w2);
     } else {
-        sweep<2, V>(Q, buf[0], buf[1], x, w0);
-        sweep<3, V>(Q, buf[1], buf[0], x, w1);
-        sweep<4, V>(Q, buf[0], buf[1], x, w2);
+        sweep<2, V, kT>(P, buf[0], buf[1], w0);
+        sweep<3, V, kT>(P, buf[1], buf[0], w1);
+        sweep<4, V, kT>(P, buf[0], buf[1], w2);
     }
 
-    // the leaf's own values: slabs and rows 4 .. 11, the two middle quads
-    const bool own = slab >= 4 && slab < 12 && ry >= 4 && ry < 12 && (qz == 1 || qz == 2);
-    if (own) stq(Xout + size_t(leaf) * 512 + row, x);
-    if (MODE == kPost) return;
-
-    // residual on the own brick, then restriction into the parent's octant;
-    // the buffer that the last sweep read holds the residual
+    // the leaf's own values: slabs and rows 4 .. 11, the two middle quads;
+    // then the residual on the own brick, in the buffer that the last sweep
+    // read, and its restriction into the parent's octant
     const float4* fin = MODE == kPreZero ? buf[0] : buf[1];
     float* rs = reinterpret_cast<float*>(MODE == kPreZero ? buf[1] : buf[0]);
-    if (slab >= 4 && slab < 12) {   // whole wavefronts: the quad exchange needs all four lanes
-        float axv[4], rv[4];
-        quad_ax(Q, fin, x, axv);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) rv[k] = ((Q.m >> k) & 1u) ? Q.b[k] - axv[k] : 0.f;
+    for (int h = 0; h < kPer; ++h) {
+        const int slab = P.slab(h);
+        if (slab < 4 || slab > 11) continue;   // whole wavefronts: the quad exchange needs all four lanes
+        const bool own = ry >= 4 && ry < 12 && (qz == 1 || qz == 2);
+        const int row = (((slab + 4) & 7) << 6) | (ly << 3) | lz;
+        if (own) stq(Xout + size_t(leaf) * 512 + row, P.x[h]);
+        if (MODE == kPost) continue;
+        float axv[4], rv[4];
+        quad_ax(P.Q[h], fin, P.at(h), P.x[h], axv);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) rv[k] = ((P.Q[h].m >> k) & 1u) ? P.Q[h].b[k] - axv[k] : 0.f;
         if (own) stq(rs + row, rv);
     }
+    if (MODE == kPost) return;
     __syncthreads();
     if (tid < 64) {
         const int ccx = tid >> 4, ccy = (tid >> 2) & 3, ccz = tid & 3;
@@ -299,26 +334,25 @@ __device__ __forceinline__ void visit_body(const LevelView& L, const V* Xin, con
     }
 }
 
+// two workgroups per CU
 template <int MODE, class V>
-__global__ __launch_bounds__(kBlkThreads) __attribute__((amdgpu_waves_per_eu(8))) void block_visit_kernel(
-    LevelView L, const V* Xin, const V* Xc, const V* B, V* Xout, V* Cv, float w0, float w1, float w2) {
-    visit_body<MODE, V, false>(L, Xin, Xc, B, Xout, Cv, w0, w1, w2, nullptr, nullptr);
+__global__ __launch_bounds__(kBlkThreads) __attribute__((amdgpu_waves_per_eu(2 * kBlkThreads / 256))) void
+block_visit_kernel(LevelView L, const V* Xin, const V* Xc, const V* B, V* Xout, V* Cv, float w0, float w1, float w2) {
+    visit_body<MODE, V, kBlkThreads, false>(L, Xin, Xc, B, Xout, Cv, w0, w1, w2, nullptr, nullptr);
 }
 
 // The coarsest solve (right-hand side Bc, solution stored into Xc by
-// workgroup 0) followed by the kPost visit of the level above it. The CG's
-// last barrier has passed when it writes its solution into cg.sp; the barrier
-// here publishes it.
+// workgroup 0) followed by the kPost visit of the level above it, on the
+// CG's thread count. The CG's last barrier has passed when it writes its
+// solution into cg.sp; the barrier here publishes it.
 template <class V, int kMaxDof>
-__global__ __launch_bounds__(kBlkThreads) void block_post_cg_kernel(LevelView L, CoarsestView C,
-                                                                    const int32_t* dof_of, const V* Bc, V* Xc,
-                                                                    const V* Xin, const V* B, V* Xout, float w0,
-                                                                    float w1, float w2) {
-    static_assert(kBlkThreads == kCgThreads, "the standalone solve's thread count");
-    __shared__ CgShared<kBlkThreads> cg;
-    coarsest_cg_block<kBlkThreads, V, kMaxDof, true>(C, Bc, blockIdx.x == 0 ? Xc : nullptr, cg);
+__global__ __launch_bounds__(kCgThreads) void block_post_cg_kernel(LevelView L, CoarsestView C, const int32_t* dof_of,
+                                                                   const V* Bc, V* Xc, const V* Xin, const V* B,
+                                                                   V* Xout, float w0, float w1, float w2) {
+    __shared__ CgShared cg;
+    coarsest_cg_block<kCgThreads, V, kMaxDof, true>(C, Bc, blockIdx.x == 0 ? Xc : nullptr, cg);
     __syncthreads();
-    visit_body<kPost, V, true>(L, Xin, nullptr, B, Xout, nullptr, w0, w1, w2, dof_of, cg.sp);
+    visit_body<kPost, V, kCgThreads, true>(L, Xin, nullptr, B, Xout, nullptr, w0, w1, w2, dof_of, cg.sp);
 }
 
 template <int MODE, class V>
@@ -352,10 +386,10 @@ hipError_t block_post_cg_t(const LevelView& L, const CoarsestView& C, const int3
     if (!L.nb27 || !dof_of || C.ndof <= 0 || C.ndof > kMaxCoarsestDof) return hipErrorInvalidValue;
     const unsigned g = unsigned(L.nleaf);
     if (C.ndof <= kCgSmallDof)
-        block_post_cg_kernel<V, kCgSmallDof><<<g, kBlkThreads, 0, s>>>(L, C, dof_of, bc, xc, x, b, x_out, w0, w1, w2);
+        block_post_cg_kernel<V, kCgSmallDof><<<g, kCgThreads, 0, s>>>(L, C, dof_of, bc, xc, x, b, x_out, w0, w1, w2);
     else
         block_post_cg_kernel<V, kMaxCoarsestDof>
-            <<<g, kBlkThreads, 0, s>>>(L, C, dof_of, bc, xc, x, b, x_out, w0, w1, w2);
+            <<<g, kCgThreads, 0, s>>>(L, C, dof_of, bc, xc, x, b, x_out, w0, w1, w2);
     return hipGetLastError();
 }
 

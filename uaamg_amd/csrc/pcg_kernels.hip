@@ -352,20 +352,20 @@ __global__ __launch_bounds__(kBlockThreads) void update_kernel(LevelView L, cons
 
 // ---------------------------------------------------------- coarsest solve
 // Workgroup size of the coarsest CG: kCgThreads by default; UAAMG_CG_THREADS = 256 or
-// 512 selects another (a tuning knob: the reductions' partial sums then group
+// 1024 selects another (a tuning knob: the reductions' partial sums then group
 // differently, so single and batched solves must run with the same setting).
 int cg_threads() {
     static const int t = [] {
         const char* e = std::getenv("UAAMG_CG_THREADS");
         const int v = e ? std::atoi(e) : kCgThreads;
-        return (v == 256 || v == 512) ? v : kCgThreads;
+        return (v == 256 || v == 1024) ? v : kCgThreads;
     }();
     return t;
 }
 
 template <class V, int kMaxDof, int kT>
 __global__ __launch_bounds__(kT) void coarsest_cg_kernel(CoarsestView C, const V* B, V* X) {
-    __shared__ CgShared<kT> sh;
+    __shared__ CgShared sh;
     coarsest_cg_block<kT, V, kMaxDof>(C, B, X, sh);
 }
 
@@ -700,7 +700,7 @@ __global__ __launch_bounds__(kFinThreads) void bstatus_kernel(int nprob, const B
 
 template <class V, int kMaxDof, int kT>
 __global__ __launch_bounds__(kT) void bcoarsest_kernel(const CoarsestView* views, const V* B, V* X) {
-    __shared__ CgShared<kT> sh;
+    __shared__ CgShared sh;
     const CoarsestView C = views[blockIdx.x];
     coarsest_cg_block<kT, V, kMaxDof>(C, B, X, sh);
 }
@@ -719,11 +719,11 @@ hipError_t launch_cg_variant(bool batched, const CoarsestView* views, const Coar
     } while (0)
     if (small) {
         if (t == 256) UAAMG_CG_LAUNCH(kCgSmallDof, 256);
-        else if (t == 512) UAAMG_CG_LAUNCH(kCgSmallDof, 512);
+        else if (t == 1024) UAAMG_CG_LAUNCH(kCgSmallDof, 1024);
         else UAAMG_CG_LAUNCH(kCgSmallDof, kCgThreads);
     } else {
-        if (t == kCgThreads) UAAMG_CG_LAUNCH(kMaxCoarsestDof, kCgThreads);
-        else UAAMG_CG_LAUNCH(kMaxCoarsestDof, 512);
+        if (t == 1024) UAAMG_CG_LAUNCH(kMaxCoarsestDof, 1024);
+        else UAAMG_CG_LAUNCH(kMaxCoarsestDof, kCgThreads);
     }
 #undef UAAMG_CG_LAUNCH
     return hipGetLastError();

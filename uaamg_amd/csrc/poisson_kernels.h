@@ -140,8 +140,8 @@ struct alignas(64) HostMailbox {
 // and the 7 stencil values in the operator's summation order.
 struct CoarsestView {
     int32_t ndof;
-    const int32_t* pos;       // [ndof] leaf*512 + offset
-    const int32_t* nb;        // [ndof][6]: +x,-x,+y,-y,+z,-z DOF index or -1
+    const int32_t* row;       // [ndof][4]: +x,-x,+y,-y,+z,-z DOF index (kMaxCoarsestDof: none) as 16-bit
+                              // pairs, low half first; leaf*512 + offset
     const float* coef;        // [ndof][8]: diag, c+x, c-x, c+y, c-y, c+z, c-z, invdiag (Eigen's 1/diag or 1)
     int32_t max_iters;        // 10 (constructCoarsestLevelExactSolver)
     float tol;                // Eigen default: float epsilon
@@ -169,12 +169,13 @@ constexpr int kBlockThreads = 64 * kWavesPerBlock;
 constexpr int kMaxCoarsestDof = 4096;
 // Workgroup size of the coarsest CG. The grouping of its sums depends on it, so
 // every kernel that solves the coarsest system (standalone, batched, inside a
-// block post-visit, in the tail kernel) uses the same. A full-size workgroup
-// keeps two rows per thread at 2048 rows, where the serial work per thread is
-// what an iteration waits for.
-constexpr int kCgThreads = 1024;
-// coarsest systems up to this size keep two row slots per thread (fewer
-// registers and less serial work than the four of the full size)
+// block post-visit, in the tail kernel) uses the same. At 1697 rows a solve
+// takes 14.2 us on 256 threads, 11.9 on 512 and 17.0 on 1024: fewer
+// wavefronts leave too much serial work per thread, more make every sum and
+// barrier longer.
+constexpr int kCgThreads = 512;
+// coarsest systems up to this size keep four row slots per thread (fewer
+// registers and less serial work than the eight of the full size)
 constexpr int kCgSmallDof = 2048;
 
 // ---- launchers (stream-ordered, no host synchronisation) ----

@@ -900,6 +900,19 @@ void coarsest_system(const PoissonLevelHost& l, int64_t leaf_offset, std::vector
     }
 }
 
+// CoarsestView::row of a system from coarsest_system
+std::vector<int32_t> coarsest_rows(const std::vector<int32_t>& pos, const std::vector<int32_t>& nb) {
+    static_assert(kMaxCoarsestDof < 65536, "16-bit neighbour indices");
+    std::vector<int32_t> rows(pos.size() * 4);
+    auto half = [](int32_t d) { return uint32_t(d >= 0 ? d : kMaxCoarsestDof); };
+    for (size_t i = 0; i < pos.size(); ++i) {
+        for (size_t k = 0; k < 3; ++k)
+            rows[i * 4 + k] = int32_t(half(nb[i * 6 + 2 * k]) | (half(nb[i * 6 + 2 * k + 1]) << 16));
+        rows[i * 4 + 3] = pos[i];
+    }
+    return rows;
+}
+
 int PoissonDevice::build_coarsest() {
     const PoissonLevelHost& l = host_.levels.back();
     const int64_t nd = l.ndof;
@@ -916,8 +929,8 @@ int PoissonDevice::build_coarsest() {
         return p;
     };
     cv_.ndof = int32_t(nd);
-    cv_.pos = static_cast<const int32_t*>(up(pos.data(), pos.size() * sizeof(int32_t)));
-    cv_.nb = static_cast<const int32_t*>(up(nb.data(), nb.size() * sizeof(int32_t)));
+    const std::vector<int32_t> rows = coarsest_rows(pos, nb);
+    cv_.row = static_cast<const int32_t*>(up(rows.data(), rows.size() * sizeof(int32_t)));
     cv_.coef = static_cast<const float*>(up(coef.data(), coef.size() * sizeof(float)));
     cv_.max_iters = 10;
     cv_.tol = FLT_EPSILON;

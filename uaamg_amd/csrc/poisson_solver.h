@@ -27,6 +27,8 @@ float scheduled_weight_iterative(int n, int i);
 // and the stencil values (diag, c+x, c-x, c+y, c-y, c+z, c-z, Eigen's invdiag).
 void coarsest_system(const PoissonLevelHost& l, int64_t leaf_offset, std::vector<int32_t>& pos,
                      std::vector<int32_t>& nb, std::vector<float>& coef);
+// positions and neighbours packed as CoarsestView::row
+std::vector<int32_t> coarsest_rows(const std::vector<int32_t>& pos, const std::vector<int32_t>& nb);
 
 struct SolverOptions {
     float relative_tolerance = 1e-7f;

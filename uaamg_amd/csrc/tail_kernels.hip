@@ -23,7 +23,7 @@ constexpr int kTailWaves = kTailThreads / 64;
 
 struct TailShared {
     float rs[kTailWaves][512];
-    CgShared<kTailThreads> cg;
+    CgShared cg;
 };
 
 __device__ __forceinline__ int first_wave_leaf() { return __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)); }
@@ -116,7 +116,7 @@ __global__ __launch_bounds__(kTailThreads) void tail_kernel(TailArgs A) {
         }
         block_residual_restrict(L, cur, A.B, A.Bc, sh.rs);
         __syncthreads();
-        coarsest_cg_block<kTailThreads>(A.C, A.Bc, A.Xc, sh.cg);
+        coarsest_cg_block<kCgThreads>(A.C, A.Bc, A.Xc, sh.cg);
         __syncthreads();
         {
             float* dst = next();
