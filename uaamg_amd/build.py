@@ -28,6 +28,7 @@ SOURCES = [
     "capi.cpp",
     "viscosity_host.cpp",
     "viscosity_kernels.hip",
+    "visc_rows_kernels.hip",
     "viscosity_solver.cpp",
     "capi_viscosity.cpp",
     "batch_solver.cpp",

@@ -247,8 +247,7 @@ int ViscBatch::init(std::vector<ViscHierarchyHost>&& probs, const ViscOptions& o
     bytes += al((D0 * 3 / kWavesPerBlock + 16) * 8);                // partials
     bytes += al(size_t(K) * sizeof(BatchPcg)) + al(64) + al(size_t(K) * sizeof(ViscCoarsestView));
     for (const auto& c : ch)
-        bytes += al(c.inv.size() * 4) + al(c.pos.size() * 4) + al(c.ecol.size() * 4) + al(c.eval.size() * 4) +
-                 al(c.elen.size() * 4);
+        bytes += al(c.inv.size() * 4) + al(c.pos.size() * 4) + al(c.epair.size() * 4) + al(c.eval.size() * 4);
 
     if (check(hipSetDevice(opt_.device), "hipSetDevice")) return -3;
     if (opt_.stream) {
@@ -345,10 +344,8 @@ int ViscBatch::init(std::vector<ViscHierarchyHost>&& probs, const ViscOptions& o
             cv.n = int32_t(c.n);
             cv.invdiag = static_cast<const float*>(up(c.inv.data(), c.inv.size() * 4));
             cv.pos = static_cast<const int32_t*>(up(c.pos.data(), c.pos.size() * 4));
-            cv.ecol = static_cast<const int32_t*>(up(c.ecol.data(), c.ecol.size() * 4));
+            cv.epair = static_cast<const uint32_t*>(up(c.epair.data(), c.epair.size() * 4));
             cv.eval = static_cast<const float*>(up(c.eval.data(), c.eval.size() * 4));
-            cv.elen = static_cast<const int32_t*>(up(c.elen.data(), c.elen.size() * 4));
-            cv.ewidth = c.width;
             cv.max_iters = 10;
             cv.tol = FLT_EPSILON;
         }

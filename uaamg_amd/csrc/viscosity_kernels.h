@@ -95,23 +95,19 @@ enum ViscMode : int { kVNormal = 0, kVResidual = 1, kVJacobi = 2, kVSpai0Mode = 
 // Eigen-CG restatement of the coarsest level on its explicit rows
 struct ViscCoarsestView {
     int32_t n;
-    const int64_t* ptr;        // [n+1]
-    const int32_t* col;        // column ascending
-    const float* val;
     const float* invdiag;      // Eigen DiagonalPreconditioner: 1/diag or 1
     const int32_t* pos;        // [n] linear index of the DOF in the level's vector
-    // the same rows as ELL, entry k of row d at [k * n + d] (columns ascending,
-    // rows padded to kViscMaxRow with value 0 and column d)
-    const int32_t* ecol;
-    const float* eval;
-    const int32_t* elen;       // [n] entries of each row
-    int32_t ewidth;            // longest row, <= kViscMaxRow
+    // the rows as ELL, entry k of row d at [k * n + d] (columns ascending, rows
+    // padded to kViscMaxRow with value 0 and column n); columns as byte offsets
+    // into a float vector, in 16-bit pairs
+    const uint32_t* epair;     // [(kViscMaxRow + 1) / 2][n], entry 2k in the low half
+    const float* eval;         // [kViscMaxRow][n]
     int32_t max_iters;
     float tol;
 };
 
 constexpr int kViscMaxCoarsest = 4096;
-constexpr int kViscMaxRow = 16;    // 1 + 6 + 8 entries per row at most
+constexpr int kViscMaxRow = 15;    // 1 + 6 + 8 entries per row at most
 
 // Level vectors are FP32, or BF16 on the coarse levels of the mixed form
 // (precision 1): loads widen exactly, stores round to nearest even, and every

@@ -5,153 +5,17 @@
 // by one, the same-channel sum ((x+ + x-) + (y+ + y-)) + (z+ + z-), then the two
 // cross-channel groups, fused multiply-adds exactly where the AVX code uses
 // _mm256_fmadd_ps (build with -ffp-contract=off).
-#include <cfloat>
-
-#include "stencil_device.h"
-#include "viscosity_host.h"
-#include "viscosity_kernels.h"
-#include "wave_reduce.h"
+#include "visc_coarsest_device.h"
+#include "viscosity_device.h"
 #include "xcd_map.h"
 
 namespace uaamg {
 namespace {
 
+using namespace dev;
+
 constexpr int kVWaves = 4;
 constexpr int kVThreads = 64 * kVWaves;
-
-constexpr int nb_slot(int ax, int ay, int az) { return (ax + 1) * 9 + (ay + 1) * 3 + (az + 1); }
-
-__device__ __forceinline__ int row_off(int X, int Y) { return ((X & 7) * 8 + (Y & 7)) * 8; }
-
-__device__ __forceinline__ void ld8v(const float* p, float v[8]) {
-    const float4 a = *reinterpret_cast<const float4*>(p);
-    const float4 b = *reinterpret_cast<const float4*>(p + 4);
-    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
-    v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-}
-__device__ __forceinline__ void st8v(float* p, const float v[8]) {
-    *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
-    *reinterpret_cast<float4*>(p + 4) = make_float4(v[4], v[5], v[6], v[7]);
-}
-// BF16-stored level vectors of the mixed form: a z-row is 16 bytes, widened
-// exactly on load, rounded to nearest even on store; arithmetic stays FP32
-__device__ __forceinline__ void ld8v(const bf16* p, float v[8]) { dev::ld8(p, v); }
-__device__ __forceinline__ void st8v(bf16* p, const float v[8]) { dev::st8(p, v); }
-__device__ __forceinline__ float ld1v(const float* p) { return *p; }
-__device__ __forceinline__ float ld1v(const bf16* p) { return float(*p); }
-__device__ __forceinline__ void st1v(float* p, float v) { *p = v; }
-__device__ __forceinline__ void st1v(bf16* p, float v) { *p = bf16(v); }
-
-// A wave record (layout at kVRecLeaf) in scalar registers.
-struct VRec {
-    int leaf;
-    int nb[27];
-    int own[14];
-    int nbs[7];
-};
-
-__device__ __forceinline__ VRec load_vrec(const ViscLevelView& L, int e) {
-    const int4* p = reinterpret_cast<const int4*>(L.wrec + size_t(e) * kVRec);
-    int v[52];
-#pragma unroll
-    for (int i = 0; i < 13; ++i) {
-        const int4 q = p[i];
-        v[4 * i] = q.x; v[4 * i + 1] = q.y; v[4 * i + 2] = q.z; v[4 * i + 3] = q.w;
-    }
-    VRec r;
-    r.leaf = v[kVRecLeaf];
-#pragma unroll
-    for (int k = 0; k < 27; ++k) r.nb[k] = v[kVRecNb + k];
-#pragma unroll
-    for (int k = 0; k < 14; ++k) r.own[k] = v[kVRecOwn + k];
-#pragma unroll
-    for (int k = 0; k < 7; ++k) r.nbs[k] = v[kVRecNbr + k];
-    // One use of every field here, in the kernel's first basic block: the
-    // record's scalar loads are then issued together and waited for once
-    // (otherwise each is issued in the branch that first reads it). The
-    // empty asm emits no instruction.
-    int all = 0;
-#pragma unroll
-    for (int k = 0; k < 49; ++k) all ^= v[k];
-    asm volatile("" ::"s"(all));
-    return r;
-}
-
-// Leaf holding leaf-local row (lx + OX, ly + OY), shifted AZ leaves in z:
-// one of four record entries chosen per lane.
-template <int OX, int OY, int AZ>
-__device__ __forceinline__ int vleaf(const VRec& R, int lx, int ly) {
-    constexpr int sx = (OX > 0) - (OX < 0), sy = (OY > 0) - (OY < 0);
-    const int X = lx + OX, Y = ly + OY;
-    const bool ox = X < 0 || X > 7, oy = Y < 0 || Y > 7;
-    const int l00 = R.nb[nb_slot(0, 0, AZ)], l10 = R.nb[nb_slot(sx, 0, AZ)];
-    const int l01 = R.nb[nb_slot(0, sy, AZ)], l11 = R.nb[nb_slot(sx, sy, AZ)];
-    return ox ? (oy ? l11 : l10) : (oy ? l01 : l00);
-}
-
-// channel ch of vector v at (lx + OX, ly + OY, z + OZ), z = 0..7 (a missing
-// leaf, or one without vector bricks, reads 0)
-template <int OX, int OY, int OZ, class V>
-__device__ __forceinline__ void vfetch(const ViscLevelView& L, const V* v, int ch, const VRec& R, int lx, int ly,
-                                       float out[8]) {
-    const int X = lx + OX, Y = ly + OY;
-    const int lf = vleaf<OX, OY, 0>(R, lx, ly);
-    float row[8];
-    if (lf >= 0 && lf < L.nleaf_dof) ld8v(v + (size_t(lf) * 3 + ch) * 512 + row_off(X, Y), row);
-    else {
-#pragma unroll
-        for (int k = 0; k < 8; ++k) row[k] = 0.f;
-    }
-    if (OZ == 0) {
-#pragma unroll
-        for (int k = 0; k < 8; ++k) out[k] = row[k];
-    } else if (OZ > 0) {
-#pragma unroll
-        for (int k = 0; k < 7; ++k) out[k] = row[k + 1];
-        const int lz = vleaf<OX, OY, 1>(R, lx, ly);
-        out[7] = (lz >= 0 && lz < L.nleaf_dof) ? ld1v(v + (size_t(lz) * 3 + ch) * 512 + row_off(X, Y)) : 0.f;
-    } else {
-#pragma unroll
-        for (int k = 7; k > 0; --k) out[k] = row[k - 1];
-        const int lz = vleaf<OX, OY, -1>(R, lx, ly);
-        out[0] = (lz >= 0 && lz < L.nleaf_dof) ? ld1v(v + (size_t(lz) * 3 + ch) * 512 + row_off(X, Y) + 7) : 0.f;
-    }
-}
-
-// coefficient grid GID at (lx + OX, ly + OY, z + OZ), at most one offset
-// nonzero: rows inside the leaf read slot s_own, rows (or the shifted z
-// value) beyond the face read s_nb; slot -1 reads the level default
-template <int GID, int OX, int OY, int OZ>
-__device__ __forceinline__ void cfetch(const ViscLevelView& L, int s_own, int s_nb, int lx, int ly, float out[8]) {
-    static_assert((OX != 0) + (OY != 0) + (OZ != 0) <= 1, "single-axis coefficient offsets");
-    const int X = lx + OX, Y = ly + OY;
-    const bool beyond = X < 0 || X > 7 || Y < 0 || Y > 7;
-    const int s = beyond ? s_nb : s_own;
-    const float m = L.dflt[GID];
-    float row[8];
-    if (s >= 0) ld8v(L.pool + size_t(s) * 512 + row_off(X, Y), row);
-    else {
-#pragma unroll
-        for (int k = 0; k < 8; ++k) row[k] = m;
-    }
-    if (OZ == 0) {
-#pragma unroll
-        for (int k = 0; k < 8; ++k) out[k] = row[k];
-    } else if (OZ > 0) {
-#pragma unroll
-        for (int k = 0; k < 7; ++k) out[k] = row[k + 1];
-        out[7] = s_nb >= 0 ? L.pool[size_t(s_nb) * 512 + row_off(X, Y)] : m;
-    } else {
-#pragma unroll
-        for (int k = 7; k > 0; --k) out[k] = row[k - 1];
-        out[0] = s_nb >= 0 ? L.pool[size_t(s_nb) * 512 + row_off(X, Y) + 7] : m;
-    }
-}
-
-template <int A>
-struct Unit {
-    static constexpr int x = A == 0, y = A == 1, z = A == 2;
-};
 
 // One row (lane) of the applier on channel C for wave record e (a DOF leaf
 // of channel C): Y = op(X, B). Every load is issued unconditionally (all in
@@ -800,226 +664,16 @@ __global__ __launch_bounds__(kVThreads) void visc_zero_kernel(uint4* v, size_t n
 }
 
 // ---------------------------------------------------------- coarsest solve
-// Eigen::ConjugateGradient<RowMajor, Upper|Lower> with the diagonal
-// preconditioner, zero guess, 10 iterations, tolerance = float epsilon
-// (construct_exact_solver / solve_exact, simd_viscosity3d.cpp:2598-2657).
-// Rows are summed in column order as Eigen's row-major product does; the
-// dot-product order of Eigen's vectorised reductions is not reproduced.
-constexpr int kCgT = 512;
-constexpr int kCgPer = kViscMaxCoarsest / kCgT;
-
-__device__ __forceinline__ float wsum(float v) { return dev::wave_sum_dpp(v); }
-
-__device__ __forceinline__ float2 bsum2(float a, float b, float (*red)[kCgT / 64][2], int& par) {
-    a = wsum(a);
-    b = wsum(b);
-    const int w = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) {
-        red[par][w][0] = a;
-        red[par][w][1] = b;
-    }
-    __syncthreads();
-    float2 t = make_float2(0.f, 0.f);
-#pragma unroll
-    for (int i = 0; i < kCgT / 64; ++i) {
-        t.x += red[par][i][0];
-        t.y += red[par][i][1];
-    }
-    par ^= 1;
-    return t;
-}
-
-// Two barriers per iteration: the reduction of <p, Ap>, and the reduction of
-// ||r||^2 and <r, z>, whose barrier also publishes the new z; the new
-// direction's product is formed as A p = A z + beta A p_old (the same vector
-// as Eigen's A p, rounded differently), so no third barrier publishes p.
 // views != null: a batch of systems, workgroup i solving views[i] (one launch
 // for the problems of a merged batch whose coarsest level is the same)
-template <class V>
-__global__ __launch_bounds__(kCgT) void visc_coarsest_kernel(ViscCoarsestView C0, const ViscCoarsestView* views,
-                                                             const V* B, V* X) {
+template <class V, int kPer>
+__global__ __launch_bounds__(kVCgThreads) void visc_coarsest_kernel(ViscCoarsestView C0, const ViscCoarsestView* views,
+                                                                    const V* B, V* X) {
     const ViscCoarsestView C = views ? views[blockIdx.x] : C0;
-    __shared__ float sz[kViscMaxCoarsest];
-    __shared__ float sq[kViscMaxCoarsest];   // A z of the thread's own rows
-    __shared__ float red[2][kCgT / 64][2];
-    int par = 0;
-    const int n = C.n, tid = threadIdx.x;
-    float x[kCgPer], r[kCgPer], z[kCgPer], p[kCgPer], q[kCgPer], inv[kCgPer];
-    float rr = 0.f, rz = 0.f;
-#pragma unroll
-    for (int j = 0; j < kCgPer; ++j) {
-        const int d = tid + j * kCgT;
-        x[j] = r[j] = z[j] = p[j] = q[j] = inv[j] = 0.f;
-        if (d < n) {
-            r[j] = ld1v(B + C.pos[d]);
-            inv[j] = C.invdiag[d];
-            rr += r[j] * r[j];
-            z[j] = inv[j] * r[j];
-            sz[d] = z[j];
-            rz += r[j] * z[j];
-        }
-    }
-    const float2 s0 = bsum2(rr, rz, red, par);   // its barrier publishes z
-    const float rhs2 = s0.x;
-    const float thr = fmaxf(C.tol * C.tol * rhs2, FLT_MIN);
-    if (rhs2 != 0.f && !(rhs2 < thr)) {
-        float abs_new = s0.y, beta = 0.f;
-        for (int it = 0; it < C.max_iters; ++it) {
-            // A z row by row: a row's entries are loaded together (padding is
-            // in bounds) and summed in column order up to the row's length;
-            // the rows loop is not unrolled (registers), so the sums go
-            // through LDS, each read back by the thread that wrote it
-#pragma unroll 1
-            for (int j = 0; j < kCgPer; ++j) {
-                const int d = tid + j * kCgT;
-                if (d >= n) break;
-                const int len = C.elen[d];
-                float t = 0.f;
-#pragma unroll
-                for (int k = 0; k < kViscMaxRow; ++k) {
-                    const size_t at = size_t(k) * size_t(n) + size_t(d);
-                    const float m = C.eval[at] * sz[C.ecol[at]];
-                    const float u = t + m;
-                    t = k < len ? u : t;
-                }
-                sq[d] = t;
-            }
-            // p = z + beta p and A p = A z + beta A p (beta = 0 on the first step)
-            float pq = 0.f;
-#pragma unroll
-            for (int j = 0; j < kCgPer; ++j) {
-                const int d = tid + j * kCgT;
-                if (d < n) {
-                    p[j] = z[j] + beta * p[j];
-                    q[j] = sq[d] + beta * q[j];
-                    pq += p[j] * q[j];
-                }
-            }
-            // the barrier also orders this step's reads of z before the writes below
-            const float alpha = abs_new / bsum2(pq, 0.f, red, par).x;
-            rr = 0.f;
-            rz = 0.f;
-#pragma unroll
-            for (int j = 0; j < kCgPer; ++j) {
-                const int d = tid + j * kCgT;
-                if (d < n) {
-                    x[j] = x[j] + alpha * p[j];
-                    r[j] = r[j] - alpha * q[j];
-                    rr += r[j] * r[j];
-                    z[j] = inv[j] * r[j];
-                    sz[d] = z[j];
-                    rz += r[j] * z[j];
-                }
-            }
-            const float2 sums = bsum2(rr, rz, red, par);
-            if (sums.x < thr) break;
-            const float abs_old = abs_new;
-            abs_new = sums.y;
-            beta = abs_new / abs_old;
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < kCgPer; ++j) {
-        const int d = tid + j * kCgT;
-        if (d < n) st1v(X + C.pos[d], x[j]);
-    }
-}
-
-// Systems of at most kCgSmallN rows keep their ELL rows in registers (two
-// rows per thread), so an iteration reads only the shared z: the same
-// products and sums, in the same order, as visc_coarsest_kernel.
-constexpr int kCgSmallN = 1024;
-
-template <class V>
-__global__ __launch_bounds__(kCgT) void visc_coarsest_small_kernel(ViscCoarsestView C0, const ViscCoarsestView* views,
-                                                                   const V* B, V* X) {
-    const ViscCoarsestView C = views ? views[blockIdx.x] : C0;
-    constexpr int kPer = kCgSmallN / kCgT;
-    __shared__ float sz[kCgSmallN];
-    __shared__ float red[2][kCgT / 64][2];
-    int par = 0;
-    const int n = C.n, tid = threadIdx.x;
-    float x[kPer], r[kPer], z[kPer], p[kPer], q[kPer], inv[kPer];
-    float ev[kPer][kViscMaxRow];
-    int ec[kPer][kViscMaxRow], len[kPer];
-    float rr = 0.f, rz = 0.f;
-#pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-        const int d = tid + j * kCgT;
-        x[j] = r[j] = z[j] = p[j] = q[j] = inv[j] = 0.f;
-        len[j] = 0;
-#pragma unroll
-        for (int k = 0; k < kViscMaxRow; ++k) {
-            ev[j][k] = 0.f;
-            ec[j][k] = 0;
-        }
-        if (d < n) {
-            len[j] = C.elen[d];
-#pragma unroll
-            for (int k = 0; k < kViscMaxRow; ++k) {
-                const size_t at = size_t(k) * size_t(n) + size_t(d);
-                ev[j][k] = C.eval[at];
-                ec[j][k] = C.ecol[at];
-            }
-            r[j] = ld1v(B + C.pos[d]);
-            inv[j] = C.invdiag[d];
-            rr += r[j] * r[j];
-            z[j] = inv[j] * r[j];
-            sz[d] = z[j];
-            rz += r[j] * z[j];
-        }
-    }
-    const float2 s0 = bsum2(rr, rz, red, par);   // its barrier publishes z
-    const float rhs2 = s0.x;
-    const float thr = fmaxf(C.tol * C.tol * rhs2, FLT_MIN);
-    if (rhs2 != 0.f && !(rhs2 < thr)) {
-        float abs_new = s0.y, beta = 0.f;
-        for (int it = 0; it < C.max_iters; ++it) {
-            float pq = 0.f;
-#pragma unroll
-            for (int j = 0; j < kPer; ++j) {
-                const int d = tid + j * kCgT;
-                if (d < n) {
-                    float t = 0.f;
-#pragma unroll
-                    for (int k = 0; k < kViscMaxRow; ++k) {
-                        const float m = ev[j][k] * sz[ec[j][k]];
-                        const float u = t + m;
-                        t = k < len[j] ? u : t;
-                    }
-                    p[j] = z[j] + beta * p[j];
-                    q[j] = t + beta * q[j];
-                    pq += p[j] * q[j];
-                }
-            }
-            // the barrier also orders this step's reads of z before the writes below
-            const float alpha = abs_new / bsum2(pq, 0.f, red, par).x;
-            rr = 0.f;
-            rz = 0.f;
-#pragma unroll
-            for (int j = 0; j < kPer; ++j) {
-                const int d = tid + j * kCgT;
-                if (d < n) {
-                    x[j] = x[j] + alpha * p[j];
-                    r[j] = r[j] - alpha * q[j];
-                    rr += r[j] * r[j];
-                    z[j] = inv[j] * r[j];
-                    sz[d] = z[j];
-                    rz += r[j] * z[j];
-                }
-            }
-            const float2 sums = bsum2(rr, rz, red, par);
-            if (sums.x < thr) break;
-            const float abs_old = abs_new;
-            abs_new = sums.y;
-            beta = abs_new / abs_old;
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-        const int d = tid + j * kCgT;
-        if (d < n) st1v(X + C.pos[d], x[j]);
-    }
+    __shared__ ViscCgShared sh;
+    __shared__ float sz[kViscMaxCoarsest + 1];
+    visc_cg_block<kPer>(
+        C, sz, sh, [&](int d) { return ld1v(B + C.pos[d]); }, [&](int d, float x) { st1v(X + C.pos[d], x); });
 }
 
 template <int MODE, class V>
@@ -1132,23 +786,27 @@ hipError_t prolong_from(const ViscLevelView& fine, const VC* coarse_v, VF* fine_
     return hipGetLastError();
 }
 
+// rows per thread by the (widest) system's size; the results do not depend on it
+template <class V>
+hipError_t coarsest_n(const ViscCoarsestView& C, const ViscCoarsestView* views, unsigned count, int max_n, const V* b,
+                      V* x, hipStream_t s) {
+    if (max_n > kViscMaxCoarsest) return hipErrorInvalidValue;
+    if (max_n <= 2 * kVCgThreads) visc_coarsest_kernel<V, 2><<<count, kVCgThreads, 0, s>>>(C, views, b, x);
+    else if (max_n <= 4 * kVCgThreads) visc_coarsest_kernel<V, 4><<<count, kVCgThreads, 0, s>>>(C, views, b, x);
+    else visc_coarsest_kernel<V, 8><<<count, kVCgThreads, 0, s>>>(C, views, b, x);
+    return hipGetLastError();
+}
+
 template <class V>
 hipError_t coarsest(const ViscCoarsestView& C, const V* b, V* x, hipStream_t s) {
     if (C.n <= 0) return hipSuccess;
-    if (C.n > kViscMaxCoarsest) return hipErrorInvalidValue;
-    if (C.n <= kCgSmallN) visc_coarsest_small_kernel<V><<<1, kCgT, 0, s>>>(C, nullptr, b, x);
-    else visc_coarsest_kernel<V><<<1, kCgT, 0, s>>>(C, nullptr, b, x);
-    return hipGetLastError();
+    return coarsest_n<V>(C, nullptr, 1, C.n, b, x, s);
 }
 
 template <class V>
 hipError_t bcoarsest(const ViscCoarsestView* views, int count, int max_n, const V* b, V* x, hipStream_t s) {
     if (count <= 0) return hipSuccess;
-    if (max_n > kViscMaxCoarsest) return hipErrorInvalidValue;
-    // the register form when every system fits it, as each problem alone would run
-    if (max_n <= kCgSmallN) visc_coarsest_small_kernel<V><<<unsigned(count), kCgT, 0, s>>>({}, views, b, x);
-    else visc_coarsest_kernel<V><<<unsigned(count), kCgT, 0, s>>>({}, views, b, x);
-    return hipGetLastError();
+    return coarsest_n<V>({}, views, unsigned(count), max_n, b, x, s);
 }
 
 template <class V>

@@ -39,6 +39,10 @@ void ViscDevice::release_device() {
     sc_ = nullptr;
     partials_ = nullptr;
     cv_ = ViscCoarsestView{};
+    rows_level_ = -1;
+    rows_ = ViscRowsView{};
+    rows_dev_ = nullptr;
+    cv_dev_ = nullptr;
     arena_.release();
 }
 
@@ -171,18 +175,17 @@ bool visc_coarsest_host(const ViscHierarchyHost& H, const int32_t* leaf_map, Vis
         err = "coarsest row longer than the stencil allows";
         return false;
     }
-    out.width = width;
     // stored at the full kViscMaxRow width, so the kernel's loads need no bound
-    out.ecol.assign(static_cast<size_t>(n) * kViscMaxRow, 0);
-    out.elen.assign(static_cast<size_t>(n), 0);
+    static_assert(kViscMaxCoarsest * 4 < 65536, "16-bit byte offsets");
+    out.epair.assign(size_t(n) * ((kViscMaxRow + 1) / 2), uint32_t(4 * n) | (uint32_t(4 * n) << 16));
     out.eval.assign(size_t(n) * kViscMaxRow, 0.f);
     for (int64_t i = 0; i < n; ++i) {
         const int64_t b = H.cptr[i], len = H.cptr[i + 1] - b;
-        out.elen[size_t(i)] = int32_t(len);
-        for (int32_t k = 0; k < kViscMaxRow; ++k) {
-            const size_t at = size_t(k) * size_t(n) + size_t(i);
-            out.ecol[at] = k < len ? H.ccol[size_t(b + k)] : int32_t(i);
-            out.eval[at] = k < len ? H.cval[size_t(b + k)] : 0.f;
+        for (int64_t k = 0; k < len; ++k) {
+            uint32_t& e = out.epair[size_t(k / 2) * size_t(n) + size_t(i)];
+            const uint32_t col = uint32_t(4 * H.ccol[size_t(b + k)]);
+            e = (k & 1) ? (e & 0xffffu) | (col << 16) : (e & 0xffff0000u) | col;
+            out.eval[size_t(k) * size_t(n) + size_t(i)] = H.cval[size_t(b + k)];
         }
     }
     return true;
@@ -197,23 +200,97 @@ int ViscDevice::build_coarsest() {
         return p;
     };
     cv_.n = int32_t(ch.n);
-    cv_.ptr = static_cast<const int64_t*>(put(host_.cptr.data(), host_.cptr.size() * 8));
-    cv_.col = static_cast<const int32_t*>(put(host_.ccol.data(), host_.ccol.size() * 4));
-    cv_.val = static_cast<const float*>(put(host_.cval.data(), host_.cval.size() * 4));
     cv_.invdiag = static_cast<const float*>(put(ch.inv.data(), ch.inv.size() * 4));
-    cv_.ewidth = ch.width;
-    cv_.ecol = static_cast<const int32_t*>(put(ch.ecol.data(), ch.ecol.size() * 4));
+    cv_.epair = static_cast<const uint32_t*>(put(ch.epair.data(), ch.epair.size() * 4));
     cv_.eval = static_cast<const float*>(put(ch.eval.data(), ch.eval.size() * 4));
-    cv_.elen = static_cast<const int32_t*>(put(ch.elen.data(), ch.elen.size() * 4));
     cv_.pos = static_cast<const int32_t*>(put(ch.pos.data(), ch.pos.size() * 4));
     cv_.max_iters = 10;
     cv_.tol = FLT_EPSILON;
-    if (!cv_.ptr || !cv_.col || !cv_.val || !cv_.invdiag || !cv_.pos || !cv_.ecol || !cv_.eval || !cv_.elen) {
+    if (!cv_.invdiag || !cv_.pos || !cv_.epair || !cv_.eval) {
         err_ = "device arena too small";
         return -2;
     }
     // the host arrays die here
     if (check(hipStreamSynchronize(stream_), "coarsest upload")) return -3;
+    return 0;
+}
+
+void visc_rows_host(const ViscLevelHost& l, int32_t start[7], std::vector<int32_t>& base) {
+    // z bits of a row with x + y even: red at even z
+    constexpr uint64_t kEven = 0x55, kOdd = 0xaa;
+    uint64_t red[2] = {0, 0};   // red bits of a mask word (one x) of even / odd x
+    for (int y = 0; y < 8; ++y) {
+        red[0] |= ((y & 1) ? kOdd : kEven) << (8 * y);
+        red[1] |= ((y & 1) ? kEven : kOdd) << (8 * y);
+    }
+    base.assign(l.nleaf_dof * 6, 0);
+    int32_t at = 0;
+    for (int c = 0; c < 3; ++c)
+        for (int colour = 0; colour < 2; ++colour) {
+            start[2 * c + colour] = at;
+            for (size_t i = 0; i < l.nleaf_dof; ++i) {
+                const size_t brick = i * 3 + size_t(c);
+                base[brick * 2 + size_t(colour)] = at;
+                for (int x = 0; x < 8; ++x) {
+                    const uint64_t m = l.mask[brick * 8 + size_t(x)];
+                    at += __builtin_popcountll(m & (colour ? ~red[x & 1] : red[x & 1]));
+                }
+            }
+        }
+    start[6] = at;
+}
+
+// Whether the level above the coarsest runs as rows: its visits then take one
+// launch instead of 30. A matter of size alone (visc_rows.h); flags bits 5 and
+// 7 and the UAAMG_VSMALL_* variables ask for the other mappings, UAAMG_VROWS=0
+// switches this one off. With two levels in the mixed form the level is FP32
+// and the coarsest BF16, which the kernel does not do.
+bool ViscDevice::wants_rows() const {
+    const int L = int(host_.levels.size());
+    if (L < 2 || (opt_.flags & (32 | 128)) || std::getenv("UAAMG_VSMALL_LEAVES") || std::getenv("UAAMG_VSMALL_TUNE"))
+        return false;
+    if (const char* env = std::getenv("UAAMG_VROWS"))
+        if (env[0] == '0') return false;
+    const int64_t n = host_.levels[size_t(L - 2)].ndof, nc = host_.levels[size_t(L - 1)].ndof;
+    return n > 0 && nc > 0 && n <= kViscRowsMax && nc <= kViscMaxCoarsest && !(L == 2 && opt_.precision == 1);
+}
+
+int ViscDevice::build_rows() {
+    if (!wants_rows()) return 0;
+    const int l = int(host_.levels.size()) - 2;
+    const ViscLevelHost& h = host_.levels[size_t(l)];
+    if (check(visc_rows_init(), "rows kernel attributes")) return -3;
+    std::vector<int32_t> base;
+    visc_rows_host(h, rows_.start, base);
+    rows_.n = rows_.start[6];
+    rows_.np = (rows_.n + 63) & ~63;
+    rows_.nc = cv_.n;
+    rows_.coef = static_cast<float4*>(arena_.take(size_t(rows_.np) * 4 * sizeof(float4)));
+    rows_.idx = static_cast<uint4*>(arena_.take(size_t(rows_.np) * 2 * sizeof(uint4)));
+    rows_.pos = static_cast<int32_t*>(arena_.take(size_t(rows_.np) * 4));
+    rows_.b = static_cast<float*>(arena_.take(size_t(rows_.np) * 4));
+    rows_.r = static_cast<float*>(arena_.take(size_t(rows_.np) * 4 + 4));
+    rows_.child = static_cast<uint4*>(arena_.take(size_t(rows_.nc) * sizeof(uint4)));
+    rows_dev_ = static_cast<ViscRowsView*>(arena_.take(sizeof(ViscRowsView)));
+    cv_dev_ = static_cast<ViscCoarsestView*>(arena_.take(sizeof(ViscCoarsestView)));
+    int32_t* base_dev = static_cast<int32_t*>(arena_.take(base.size() * 4));
+    if (!rows_.coef || !rows_.idx || !rows_.pos || !rows_.b || !rows_.r || !rows_.child || !rows_dev_ || !cv_dev_ ||
+        !base_dev) {
+        err_ = "device arena too small";
+        return -2;
+    }
+    check(hipMemcpyAsync(rows_dev_, &rows_, sizeof(rows_), hipMemcpyHostToDevice, stream_), "upload");
+    check(hipMemcpyAsync(cv_dev_, &cv_, sizeof(cv_), hipMemcpyHostToDevice, stream_), "upload");
+    check(hipMemcpyAsync(base_dev, base.data(), base.size() * 4, hipMemcpyHostToDevice, stream_), "upload");
+    // the row maps use two PCG vectors as scratch, which go back to zero
+    check(launch_visc_rows_build(lv_[size_t(l)].v, lv_[size_t(l) + 1].v, rows_, base_dev, cv_.pos, z0_, p0_, stream_),
+          "rows");
+    const size_t vec0 = host_.levels[0].nleaf_dof * 3 * 512 * 4;
+    check(hipMemsetAsync(z0_, 0, vec0, stream_), "memset");
+    check(hipMemsetAsync(p0_, 0, vec0, stream_), "memset");
+    if (check(hipStreamSynchronize(stream_), "rows upload")) return -3;   // base dies here
+    if (first_error_ != hipSuccess) return -3;
+    rows_level_ = l;
     return 0;
 }
 
@@ -243,10 +320,12 @@ size_t ViscDevice::device_bytes() const {
     const size_t vec0 = l0.nleaf_dof * 3 * 512 * 4;
     const size_t ndof0 = size_t(l0.ndof);
     bytes += 5 * align_up(vec0) + 3 * align_up(ndof0 * 4 + 4);
-    bytes += align_up(host_.cptr.size() * 8) + align_up(host_.ccol.size() * 4) + 3 * align_up(host_.cval.size() * 4) +
-             8 * kAlign;
     const size_t nc = size_t(host_.levels.back().ndof);
-    bytes += 2 * align_up(nc * kViscMaxRow * 4) + align_up(nc * 4) + 2 * kAlign;   // ELL rows
+    bytes += 2 * align_up(nc * (kViscMaxRow + 1) * 4) + 2 * align_up(nc * 4) + 4 * kAlign;   // coarsest rows
+    if (wants_rows()) {
+        const ViscLevelHost& lr = host_.levels[host_.levels.size() - 2];
+        bytes += visc_rows_bytes(lr.ndof, int64_t(nc)) + align_up(lr.nleaf_dof * 6 * 4) + 4 * kAlign;
+    }
     bytes += align_up(sizeof(PcgScalars)) + align_up((l0.nleaf_dof * 3 / kWavesPerBlock + 2) * 8);
     return bytes;
 }
@@ -334,6 +413,7 @@ int ViscDevice::acquire_device() {
     mailbox_->word = 0;
     if (check(hipHostGetDevicePointer(reinterpret_cast<void**>(&mailbox_dev_), mailbox_, 0), "mailbox map")) return -3;
     if (int rc = build_coarsest()) return rc;
+    if (int rc = build_rows()) return rc;
     if (check(hipStreamSynchronize(stream_), "init sync")) return -3;
     clock.lap("viscosity device: vectors + coarsest");
     if (tune) tune_levels();
@@ -457,8 +537,18 @@ void ViscDevice::rbgs(int level, V* x, const V* b, bool xyz) {
 // above the coarsest the second visit would solve the same right-hand side
 // from zero again (solve_exact starts from a zero guess) and is skipped.
 template <class V>
+void ViscDevice::rows_visit(V* x, const V* b, bool precon, int nvisits) {
+    check(launch_visc_rows_visit(rows_dev_, cv_dev_, 1, rows_.n, rows_.nc, b, x, precon, nvisits, stream_),
+          "rows visit");
+}
+
+template <class V>
 void ViscDevice::mucycle(int level, V* x, const V* b, bool precon) {
     const int L = int(lv_.size());
+    if (level == rows_level_) {   // a two-level hierarchy: the whole W-cycle
+        rows_visit<V>(x, b, precon, 1);
+        return;
+    }
     if (level == L - 1) {
         check(launch_visc_coarsest(cv_, b, x, stream_), "coarsest");
         return;
@@ -483,8 +573,12 @@ void ViscDevice::mucycle(int level, V* x, const V* b, bool precon) {
     auto below = [&](auto* cX, auto* cB) {
         using VC = std::remove_pointer_t<decltype(cX)>;
         check(launch_visc_restrict(c.v, v, static_cast<const V*>(T), cB, stream_), "restrict");
-        mucycle<VC>(level + 1, cX, cB, true);
-        if (level + 1 < L - 1) mucycle<VC>(level + 1, cX, cB, false);
+        if (level + 1 == rows_level_) {
+            rows_visit<VC>(cX, cB, true, 2);   // both visits of the level, one launch
+        } else {
+            mucycle<VC>(level + 1, cX, cB, true);
+            if (level + 1 < L - 1) mucycle<VC>(level + 1, cX, cB, false);
+        }
         check(launch_visc_prolong(v, c.v, static_cast<const VC*>(cX), x, stream_), "prolong");
     };
     if constexpr (std::is_same_v<V, bf16>) {

@@ -13,6 +13,7 @@
 #include "poisson_solver.h"
 #include "stream_order.h"
 #include "viscosity_host.h"
+#include "visc_rows.h"
 #include "viscosity_kernels.h"
 
 namespace uaamg {
@@ -39,10 +40,13 @@ std::vector<int32_t> visc_wave_records(const ViscLevelHost& h);
 // at i). False with err set when the system exceeds the kernel's limits.
 struct ViscCoarsestHost {
     int64_t n = 0;
-    int32_t width = 0;
     std::vector<float> inv, eval;
-    std::vector<int32_t> pos, ecol, elen;
+    std::vector<uint32_t> epair;
+    std::vector<int32_t> pos;
 };
+// The rows of level l (ViscRowsView): group starts, and per brick (leaf *
+// 3 + channel) the first row of its red and of its black DOFs.
+void visc_rows_host(const ViscLevelHost& l, int32_t start[7], std::vector<int32_t>& base);
 bool visc_coarsest_host(const ViscHierarchyHost& h, const int32_t* leaf_map, ViscCoarsestHost& out,
                         std::string& err);
 
@@ -117,8 +121,12 @@ private:
     int upload_level(const ViscLevelHost& h, DevLevel& d);
     int upload_spai0(int level);
     int build_coarsest();
+    int build_rows();
     template <class V>
     void rbgs(int level, V* x, const V* b, bool xyz);
+    bool wants_rows() const;
+    template <class V>
+    void rows_visit(V* x, const V* b, bool precon, int nvisits);
     template <class V>
     void mucycle(int level, V* x, const V* b, bool precon);
     template <class V>
@@ -150,6 +158,11 @@ private:
     PcgScalars* sc_ = nullptr;
     double* partials_ = nullptr;
     ViscCoarsestView cv_{};
+    // the level above the coarsest as rows, its visits as one launch (-1: per pass)
+    int rows_level_ = -1;
+    ViscRowsView rows_{};
+    ViscRowsView* rows_dev_ = nullptr;
+    ViscCoarsestView* cv_dev_ = nullptr;
     std::vector<float*> spai0_bufs_;
     Graph g_init_, g_first_, g_iter_;
     bool graphs_ready_ = false;
