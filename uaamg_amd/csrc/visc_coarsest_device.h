@@ -28,17 +28,19 @@ struct ViscCgShared {
 // Solves the system for the right-hand side ld(d) and hands the solution to
 // st(d, x); sz has room for C.n + 1 floats. Row d belongs to thread d %
 // kVCgThreads, C.n <= kPer * kVCgThreads (a larger kPer only adds empty rows).
-// Every thread of the kVCgThreads-thread block must call it; on return no
-// thread reads sz any more.
+// Every thread of the block, of kVCgThreads threads or more, must call it (the
+// threads beyond only take part in the barriers); on return no thread reads sz
+// any more.
 template <int kPer, class Load, class Store>
 __device__ __forceinline__ void visc_cg_block(const ViscCoarsestView& C, float* sz, ViscCgShared& sh, const Load& ld,
                                               const Store& st) {
     constexpr int kPairs = (kViscMaxRow + 1) / 2;
-    const int n = C.n, tid = threadIdx.x;
+    const int tid = threadIdx.x, size = C.n;
+    const int n = tid < kVCgThreads ? size : 0;   // rows d < n
     float ev[kPer][kViscMaxRow], inv[kPer], x[kPer], r[kPer], p[kPer], q[kPer];
     uint32_t ep[kPer][kPairs];
     int par = 0;
-    if (tid == 0) sz[n] = 0.f;
+    if (tid == 0) sz[size] = 0.f;
 #pragma unroll
     for (int j = 0; j < kPer; ++j) {
         const int d = tid + j * kVCgThreads;
@@ -49,9 +51,9 @@ __device__ __forceinline__ void visc_cg_block(const ViscCoarsestView& C, float* 
         for (int k = 0; k < kPairs; ++k) ep[j][k] = 0;
         if (d < n) {
 #pragma unroll
-            for (int k = 0; k < kViscMaxRow; ++k) ev[j][k] = C.eval[size_t(k) * size_t(n) + size_t(d)];
+            for (int k = 0; k < kViscMaxRow; ++k) ev[j][k] = C.eval[size_t(k) * size_t(size) + size_t(d)];
 #pragma unroll
-            for (int k = 0; k < kPairs; ++k) ep[j][k] = C.epair[size_t(k) * size_t(n) + size_t(d)];
+            for (int k = 0; k < kPairs; ++k) ep[j][k] = C.epair[size_t(k) * size_t(size) + size_t(d)];
             inv[j] = C.invdiag[d];
             r[j] = ld(d);
             sz[d] = inv[j] * r[j];
@@ -89,10 +91,12 @@ __device__ __forceinline__ void visc_cg_block(const ViscCoarsestView& C, float* 
                 zw = fmaf(z, t, zw);
             }
         }
-        rr = wave_sum_dpp(rr);
-        rz = wave_sum_dpp(rz);
-        zw = wave_sum_dpp(zw);
-        if ((tid & 63) == 0) sh.red[par][tid >> 6] = make_float4(rr, rz, zw, 0.f);
+        if ((tid >> 6) < kVCgThreads / 64) {
+            rr = wave_sum_dpp(rr);
+            rz = wave_sum_dpp(rz);
+            zw = wave_sum_dpp(zw);
+            if ((tid & 63) == 0) sh.red[par][tid >> 6] = make_float4(rr, rz, zw, 0.f);
+        }
         __syncthreads();   // also orders this step's reads of z before the writes below
         float3 s = make_float3(0.f, 0.f, 0.f);
 #pragma unroll

@@ -22,16 +22,31 @@ struct ViscRowsView {
     float4* coef = nullptr;    // [4][np]: the 14 couplings in the operator's order, 1/diag, diag
     uint4* idx = nullptr;      // [2][np]: 16-bit row numbers of the 14 neighbours (n: none), the coarse row (nc: none)
     int32_t* pos = nullptr;    // [n] position in the level vector
+    int32_t nsteps = 0;        // steps of one sweep
+    int2* steps = nullptr;     // [2][nsteps]: the steps of an XYZ and of a ZYX sweep (visc_rows_steps)
     float* b = nullptr;        // [n] scratch: right-hand side by row
     float* r = nullptr;        // [n + 1] scratch: residual by row (the last stays 0)
     uint4* child = nullptr;    // [nc] 16-bit row numbers of a coarse row's eight children (n: none)
 };
 
-// Rows the kernel takes: x and the coarsest vector fit a workgroup's LDS, and
-// row numbers fit 16 bits. A colour pass over N rows streams 100 N / 6 bytes
-// through one CU, so the time per pass grows with N while the launched passes
-// stay at about 5 us.
-constexpr int64_t kViscRowsMax = 32768;
+// Rows the kernel takes (x and the coarsest vector fit a workgroup's LDS, row
+// numbers fit 16 bits). A colour pass over N rows streams 100 N / 6 bytes
+// through one CU, so its time grows with N while the launched passes stay at
+// about 5 us. Whole solves, rows / launches, with this level at 7428 rows: 677
+// / 993 us, 11.9k: 1109 / 1507, 15.9k: 1379 / 1561, 19.0k: 1467 / 1622, 22.5k:
+// 1662 / 1714, 25.0k: 1761 / 1730.
+constexpr int64_t kViscRowsMax = 20480;
+
+// Threads of a visit's workgroup and rows per step: 1024 where the coarsest
+// rows fit 128 registers a thread (two of them), 512 beyond. Steps of one launch
+// have one size, so a batch goes by its largest coarsest level.
+constexpr int kViscRowsWideNc = 1024;
+inline int visc_rows_step(int max_nc) { return max_nc <= kViscRowsWideNc ? 1024 : 512; }
+
+// A step is up to that many rows of one group: {first row, the group's end,
+// plus kViscStepLast on a pass's last step (a barrier follows)}.
+constexpr int kViscStepLast = 1 << 30;
+constexpr int kViscMaxSteps = int(kViscRowsMax) / 512 + 6;
 
 // allows the visit kernels the LDS of the largest level; before the first visit on a device
 hipError_t visc_rows_init();

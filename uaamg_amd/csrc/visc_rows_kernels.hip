@@ -10,7 +10,8 @@ namespace {
 
 using namespace dev;
 
-constexpr int kRowThreads = kVCgThreads;
+constexpr int kStepLast = kViscStepLast;
+constexpr int kMaxSteps = kViscMaxSteps;
 
 // ------------------------------------------------------------------ build
 // Maps hold row number + 1 as a float per brick entry (0: no DOF), so the
@@ -176,20 +177,36 @@ __device__ __forceinline__ float stored(float v) {
     else return float(V(v));
 }
 
+// The views come from memory, so their pointers are generic to the compiler:
+// its flat loads would count as LDS accesses too and each barrier would wait
+// for them. Loads and stores here name the global address space.
+typedef float vf4 __attribute__((ext_vector_type(4)));
+typedef uint32_t vu4 __attribute__((ext_vector_type(4)));
+#define UAAMG_GLOBAL __attribute__((address_space(1)))
+template <class T>
+__device__ __forceinline__ T gload(const void* base, uint32_t byte) {
+    return *reinterpret_cast<const UAAMG_GLOBAL T*>((const UAAMG_GLOBAL char*)base + byte);
+}
+template <class T>
+__device__ __forceinline__ void gstore(void* base, uint32_t byte, T v) {
+    *reinterpret_cast<UAAMG_GLOBAL T*>((UAAMG_GLOBAL char*)base + byte) = v;
+}
+
 // one row's operands
 struct Row {
-    float4 c[4];
-    uint4 i[2];
+    vf4 c[4];
+    vu4 i[2];
     float b;
 };
 
 __device__ __forceinline__ Row load_row(const ViscRowsView& R, int row) {
     Row q;
+    const uint32_t o16 = uint32_t(row) * 16u;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) q.c[k] = R.coef[size_t(k) * size_t(R.np) + size_t(row)];
+    for (int k = 0; k < 4; ++k) q.c[k] = gload<vf4>(R.coef + size_t(k) * size_t(R.np), o16);
 #pragma unroll
-    for (int k = 0; k < 2; ++k) q.i[k] = R.idx[size_t(k) * size_t(R.np) + size_t(row)];
-    q.b = R.b[row];
+    for (int k = 0; k < 2; ++k) q.i[k] = gload<vu4>(R.idx + size_t(k) * size_t(R.np), o16);
+    q.b = gload<float>(R.b, uint32_t(row) * 4u);
     return q;
 }
 
@@ -217,67 +234,82 @@ __device__ __forceinline__ float row_sum(const Row& q, const float* xs) {
     return s;
 }
 
-// One colour pass over group g, x in LDS. `cur` holds the thread's first row
-// of the group; on return it holds its first row of group `next`: a row's
-// loads do not depend on x, so they are issued one row ahead, across the
-// barrier between passes too.
-template <class V>
-__device__ __forceinline__ void colour_pass(const ViscRowsView& R, const int* start, float* xs, int g, int next,
-                                            Row& cur) {
-    const int end = start[g + 1];
-    int row = start[g] + int(threadIdx.x);
-    for (;;) {
-        const bool more = row + kRowThreads < end;
-        const int ahead = more ? row + kRowThreads : start[next] + int(threadIdx.x);
-        const Row nxt = load_row(R, ahead < R.n ? ahead : 0);
-        if (row < end) {
-            float t = cur.b - row_sum(cur, xs);
-            t = t * cur.c[3].z;
-            xs[row] = stored<V>(fmaf(xs[row], 0.0f, t));
+// Rows in flight per thread: a row's operands do not depend on x, so they are
+// loaded this many steps ahead, across the barriers between passes too. (At
+// 6018 rows one, two and three ahead take the same time: what is left of a
+// pass is the CU's own work, 100 KB of rows, 14 LDS reads and about 90 vector
+// instructions a row.)
+constexpr int kRowsAhead = 2;
+
+// `sweeps` Gauss-Seidel sweeps (six colour passes each) over the steps of one
+// direction (ViscRowsView::steps, in LDS), then, with RESIDUAL, the residual
+// of every row into R.r; x in LDS.
+template <class V, bool RESIDUAL>
+__device__ __forceinline__ void run_passes(const ViscRowsView& R, const int2* steps, int nsteps, float* xs,
+                                           int sweeps) {
+    const int tid = threadIdx.x;
+    const int gs = sweeps * nsteps, total = gs + (RESIDUAL ? nsteps : 0);
+    Row buf[kRowsAhead];
+    int2 st[kRowsAhead];
+    int ahead = 0;   // the step to fetch next, modulo nsteps
+    auto fetch = [&](int u) {
+        st[u] = steps[ahead];
+        ahead = ahead + 1 < nsteps ? ahead + 1 : 0;
+        const int row = st[u].x + tid;
+        buf[u] = load_row(R, row < R.n ? row : 0);
+    };
+#pragma unroll
+    for (int u = 0; u < kRowsAhead; ++u) fetch(u);
+#pragma unroll 1
+    for (int i = 0; i < total; i += kRowsAhead) {
+#pragma unroll
+        for (int u = 0; u < kRowsAhead; ++u) {
+            if (i + u >= total) break;
+            const int row = st[u].x + tid, end = st[u].y & (kStepLast - 1);
+            const bool last = __builtin_amdgcn_readfirstlane(st[u].y) >= kStepLast;
+            if (row < end) {
+                const float s = row_sum(buf[u], xs);
+                if (!RESIDUAL || i + u < gs) {
+                    float t = buf[u].b - s;
+                    t = t * buf[u].c[3].z;
+                    xs[row] = stored<V>(fmaf(xs[row], 0.0f, t));
+                } else {
+                    gstore<float>(R.r, uint32_t(row) * 4u, stored<V>(buf[u].b - fmaf(xs[row], buf[u].c[3].w, s)));
+                }
+            }
+            fetch(u);
+            if (last) __syncthreads();
         }
-        cur = nxt;
-        if (!more) break;
-        row += kRowThreads;
     }
-    __syncthreads();
 }
 
-// The visits (see visc_rows.h). Bounded by one CU's rate of reading rows:
-// 96 + 4 bytes per row and pass, five passes over all rows per visit.
-template <class V, int kPer>
+// The visits (see visc_rows.h). Bounded by one CU's rates: 96 + 4 bytes per
+// row, five times over all rows per visit. Two visits of a 6018-row level with
+// the coarsest solves (934 rows) take 95 us; as launches a visit took 155 us.
+template <class V, int kPer, int kT>
 __device__ __forceinline__ void rows_visit(const ViscRowsView& R, const ViscCoarsestView& C, const V* B, V* X,
                                            bool precon, int nvisits) {
     extern __shared__ float sm[];
     __shared__ ViscCgShared cg;
-    __shared__ int start[7];
     float* xs = sm;                // [n + 1], the last zero
     float* sz = sm + R.n + 1;      // [nc + 1], the last zero
     const int tid = threadIdx.x;
+    __shared__ int2 steps[2 * kMaxSteps];
+    const int nsteps = R.nsteps;
+    for (int i = tid; i < 2 * nsteps; i += kT) steps[i] = make_int2(gload<int>(R.steps, uint32_t(i) * 8u), gload<int>(R.steps, uint32_t(i) * 8u + 4u));
     if (tid == 0) {
-#pragma unroll
-        for (int g = 0; g < 7; ++g) start[g] = R.start[g];
         xs[R.n] = 0.f;
-        R.r[R.n] = 0.f;
+        gstore<float>(R.r, uint32_t(R.n) * 4u, 0.f);
     }
-    for (int row = tid; row < R.n; row += kRowThreads) {
-        const int p = R.pos[row];
-        R.b[row] = ld1v(B + p);
+    for (int row = tid; row < R.n; row += kT) {
+        const int p = gload<int>(R.pos, uint32_t(row) * 4u);
+        gstore<float>(R.b, uint32_t(row) * 4u, ld1v(B + p));
         xs[row] = precon ? 0.f : ld1v(X + p);
     }
     __syncthreads();
 #pragma unroll 1
     for (int v = 0; v < nvisits; ++v) {
-        Row cur = load_row(R, tid < R.n ? tid : 0);
-#pragma unroll 1
-        for (int k = 0; k < 12; ++k) colour_pass<V>(R, start, xs, k % 6, (k + 1) % 6, cur);
-        // residual of every row
-        for (int row = tid; row < R.n; row += kRowThreads) {
-            const Row nxt = load_row(R, row + kRowThreads < R.n ? row + kRowThreads : 0);
-            const float ax = fmaf(xs[row], cur.c[3].w, row_sum(cur, xs));
-            R.r[row] = stored<V>(cur.b - ax);
-            cur = nxt;
-        }
-        __syncthreads();
+        run_passes<V, true>(R, steps, nsteps, xs, 2);
         // restriction into the coarsest solve, whose solution stays in sz (the
         // empty asm keeps its rows' loads inside the loop over visits)
         ViscCoarsestView Cv = C;
@@ -289,12 +321,11 @@ __device__ __forceinline__ void rows_visit(const ViscRowsView& R, const ViscCoar
         visc_cg_block<kPer>(
             Cv, sz, cg,
             [&](int d) {
-                const uint4 ch = R.child[d];
-                float sum = 0.f;
-                const uint32_t w[4] = {ch.x, ch.y, ch.z, ch.w};
-                float f[8];
+                const vu4 w = gload<vu4>(R.child, uint32_t(d) * 16u);
+                float sum = 0.f, f[8];
 #pragma unroll
-                for (int k = 0; k < 8; ++k) f[k] = R.r[(k & 1) ? (w[k >> 1] >> 16) : (w[k >> 1] & 0xffffu)];
+                for (int k = 0; k < 8; ++k)
+                    f[k] = gload<float>(R.r, 4u * ((k & 1) ? (w[k >> 1] >> 16) : (w[k >> 1] & 0xffffu)));
 #pragma unroll
                 for (int k = 0; k < 8; ++k) sum += f[k];
                 return stored<V>(sum * 0.125f * 0.5f * 2.0f);
@@ -302,29 +333,21 @@ __device__ __forceinline__ void rows_visit(const ViscRowsView& R, const ViscCoar
             [&](int d, float x) { sz[d] = stored<V>(x); });
         __syncthreads();
         // prolongation
-        for (int row = tid; row < R.n; row += kRowThreads)
-            xs[row] = stored<V>(xs[row] + sz[R.idx[size_t(R.np) + size_t(row)].w & 0xffffu]);
-        cur = load_row(R, start[5] + tid < R.n ? start[5] + tid : 0);
+        for (int row = tid; row < R.n; row += kT)
+            xs[row] = stored<V>(xs[row] + sz[gload<uint32_t>(R.idx + size_t(R.np), uint32_t(row) * 16u + 12u) & 0xffffu]);
         __syncthreads();
-#pragma unroll 1
-        for (int k = 0; k < 12; ++k) colour_pass<V>(R, start, xs, 5 - k % 6, 5 - (k + 1) % 6, cur);
+        run_passes<V, false>(R, steps + nsteps, nsteps, xs, 2);
     }
-    for (int row = tid; row < R.n; row += kRowThreads) st1v(X + R.pos[row], xs[row]);
+    for (int row = tid; row < R.n; row += kT) st1v(X + gload<int>(R.pos, uint32_t(row) * 4u), xs[row]);
 }
 
 // workgroup i: problem i
-template <class V, int kPer>
-__global__ __launch_bounds__(kRowThreads) void visc_rows_visit_kernel(const ViscRowsView* __restrict__ views,
-                                                                      const ViscCoarsestView* __restrict__ cviews, const V* B, V* X,
-                                                                      int precon, int nvisits) {
-    rows_visit<V, kPer>(views[blockIdx.x], cviews[blockIdx.x], B, X, precon != 0, nvisits);
-}
-
-template <class V, int kPer>
-hipError_t visit_per(const ViscRowsView* views, const ViscCoarsestView* cviews, unsigned count, size_t lds, const V* b,
-                     V* x, bool precon, int nvisits, hipStream_t s) {
-    visc_rows_visit_kernel<V, kPer><<<count, kRowThreads, lds, s>>>(views, cviews, b, x, precon ? 1 : 0, nvisits);
-    return hipGetLastError();
+template <class V, int kPer, int kT>
+__global__ __launch_bounds__(kT) void visc_rows_visit_kernel(const ViscRowsView* views, const ViscCoarsestView* cviews,
+                                                             const V* B, V* X, int precon, int nvisits) {
+    const ViscRowsView R = views[blockIdx.x];
+    const ViscCoarsestView C = cviews[blockIdx.x];
+    rows_visit<V, kPer, kT>(R, C, B, X, precon != 0, nvisits);
 }
 
 template <class V>
@@ -335,21 +358,27 @@ hipError_t visit(const ViscRowsView* views, const ViscCoarsestView* cviews, int 
         return hipErrorInvalidValue;
     const size_t lds = (size_t(max_n) + size_t(max_nc) + 2) * sizeof(float);
     const unsigned g = unsigned(count);
-    if (max_nc <= 2 * kVCgThreads) return visit_per<V, 2>(views, cviews, g, lds, b, x, precon, nvisits, s);
-    if (max_nc <= 4 * kVCgThreads) return visit_per<V, 4>(views, cviews, g, lds, b, x, precon, nvisits, s);
-    return visit_per<V, 8>(views, cviews, g, lds, b, x, precon, nvisits, s);
+    const int p = precon ? 1 : 0;
+    static_assert(2 * kVCgThreads == kViscRowsWideNc, "the wide form's coarsest size");
+    if (visc_rows_step(max_nc) == 1024)
+        visc_rows_visit_kernel<V, 2, 1024><<<g, 1024, lds, s>>>(views, cviews, b, x, p, nvisits);
+    else if (max_nc <= 4 * kVCgThreads)
+        visc_rows_visit_kernel<V, 4, 512><<<g, 512, lds, s>>>(views, cviews, b, x, p, nvisits);
+    else
+        visc_rows_visit_kernel<V, 8, 512><<<g, 512, lds, s>>>(views, cviews, b, x, p, nvisits);
+    return hipGetLastError();
 }
 
 }  // namespace
 
 hipError_t visc_rows_init() {
     const int most = int((kViscRowsMax + kViscMaxCoarsest + 2) * sizeof(float));
-    const void* kernels[] = {reinterpret_cast<const void*>(&visc_rows_visit_kernel<float, 2>),
-                             reinterpret_cast<const void*>(&visc_rows_visit_kernel<float, 4>),
-                             reinterpret_cast<const void*>(&visc_rows_visit_kernel<float, 8>),
-                             reinterpret_cast<const void*>(&visc_rows_visit_kernel<bf16, 2>),
-                             reinterpret_cast<const void*>(&visc_rows_visit_kernel<bf16, 4>),
-                             reinterpret_cast<const void*>(&visc_rows_visit_kernel<bf16, 8>)};
+    const void* kernels[] = {reinterpret_cast<const void*>(&visc_rows_visit_kernel<float, 2, 1024>),
+                             reinterpret_cast<const void*>(&visc_rows_visit_kernel<float, 4, 512>),
+                             reinterpret_cast<const void*>(&visc_rows_visit_kernel<float, 8, 512>),
+                             reinterpret_cast<const void*>(&visc_rows_visit_kernel<bf16, 2, 1024>),
+                             reinterpret_cast<const void*>(&visc_rows_visit_kernel<bf16, 4, 512>),
+                             reinterpret_cast<const void*>(&visc_rows_visit_kernel<bf16, 8, 512>)};
     for (const void* k : kernels)
         if (hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, most)) return e;
     return hipSuccess;
@@ -358,7 +387,8 @@ hipError_t visc_rows_init() {
 size_t visc_rows_bytes(int64_t n, int64_t nc) {
     const size_t np = (size_t(n) + 63) & ~size_t(63);
     // coef, idx, pos, b, r, child, each rounded up to an allocation unit
-    return np * (4 * sizeof(float4) + 2 * sizeof(uint4) + 3 * 4) + 256 + size_t(nc) * sizeof(uint4) + 6 * 256;
+    return np * (4 * sizeof(float4) + 2 * sizeof(uint4) + 3 * 4) + 256 + size_t(nc) * sizeof(uint4) + 2 * kMaxSteps * sizeof(int2) +
+           7 * 256;
 }
 
 hipError_t launch_visc_rows_build(const ViscLevelView& F, const ViscLevelView& Cl, const ViscRowsView& R,

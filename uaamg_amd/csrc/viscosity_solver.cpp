@@ -240,6 +240,19 @@ void visc_rows_host(const ViscLevelHost& l, int32_t start[7], std::vector<int32_
     start[6] = at;
 }
 
+std::vector<int2> visc_rows_steps(const int32_t start[7], int step) {
+    std::vector<int2> out;
+    for (int back = 0; back < 2; ++back)
+        for (int k = 0; k < 6; ++k) {
+            const int g = back ? 5 - k : k;
+            for (int32_t row = start[g]; row < start[g + 1]; row += step) {
+                const bool last = row + step >= start[g + 1];
+                out.push_back(make_int2(row, start[g + 1] + (last ? kViscStepLast : 0)));
+            }
+        }
+    return out;
+}
+
 // Whether the level above the coarsest runs as rows: its visits then take one
 // launch instead of 30. A matter of size alone (visc_rows.h); flags bits 5 and
 // 7 and the UAAMG_VSMALL_* variables ask for the other mappings, UAAMG_VROWS=0
@@ -273,14 +286,19 @@ int ViscDevice::build_rows() {
     rows_.child = static_cast<uint4*>(arena_.take(size_t(rows_.nc) * sizeof(uint4)));
     rows_dev_ = static_cast<ViscRowsView*>(arena_.take(sizeof(ViscRowsView)));
     cv_dev_ = static_cast<ViscCoarsestView*>(arena_.take(sizeof(ViscCoarsestView)));
+    const std::vector<int2> steps = visc_rows_steps(rows_.start, visc_rows_step(rows_.nc));
+    rows_.nsteps = int32_t(steps.size() / 2);
+    rows_.steps = static_cast<int2*>(arena_.take(steps.size() * sizeof(int2)));
     int32_t* base_dev = static_cast<int32_t*>(arena_.take(base.size() * 4));
-    if (!rows_.coef || !rows_.idx || !rows_.pos || !rows_.b || !rows_.r || !rows_.child || !rows_dev_ || !cv_dev_ ||
-        !base_dev) {
+    if (!rows_.coef || !rows_.idx || !rows_.pos || !rows_.b || !rows_.r || !rows_.child || !rows_.steps || !rows_dev_ ||
+        !cv_dev_ || !base_dev) {
         err_ = "device arena too small";
         return -2;
     }
     check(hipMemcpyAsync(rows_dev_, &rows_, sizeof(rows_), hipMemcpyHostToDevice, stream_), "upload");
     check(hipMemcpyAsync(cv_dev_, &cv_, sizeof(cv_), hipMemcpyHostToDevice, stream_), "upload");
+    check(hipMemcpyAsync(rows_.steps, steps.data(), steps.size() * sizeof(int2), hipMemcpyHostToDevice, stream_),
+          "upload");
     check(hipMemcpyAsync(base_dev, base.data(), base.size() * 4, hipMemcpyHostToDevice, stream_), "upload");
     // the row maps use two PCG vectors as scratch, which go back to zero
     check(launch_visc_rows_build(lv_[size_t(l)].v, lv_[size_t(l) + 1].v, rows_, base_dev, cv_.pos, z0_, p0_, stream_),

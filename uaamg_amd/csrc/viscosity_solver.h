@@ -47,6 +47,8 @@ struct ViscCoarsestHost {
 // The rows of level l (ViscRowsView): group starts, and per brick (leaf *
 // 3 + channel) the first row of its red and of its black DOFs.
 void visc_rows_host(const ViscLevelHost& l, int32_t start[7], std::vector<int32_t>& base);
+// the steps of an XYZ sweep (red, black of channel 0, 1, 2) and then of a ZYX one (ViscRowsView::steps)
+std::vector<int2> visc_rows_steps(const int32_t start[7], int step);
 bool visc_coarsest_host(const ViscHierarchyHost& h, const int32_t* leaf_map, ViscCoarsestHost& out,
                         std::string& err);
 
