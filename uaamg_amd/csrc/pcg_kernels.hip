@@ -270,18 +270,23 @@ __device__ __forceinline__ void fin_max(const double* part, int n, float& v, int
 __global__ __launch_bounds__(kFinThreads) void finalize_kernel(int op, int n, const double* partials,
                                                                PcgScalars* sc, HostMailbox* mb) {
     if (op == kFinNu) {
-        __shared__ float tv[kFinThreads];
-        __shared__ int tb[kFinThreads];
+        __shared__ float tv[kFinThreads / 64];
+        __shared__ int tb[kFinThreads / 64];
         float v;
         int b;
         fin_max(partials, n, v, b);
-        tv[threadIdx.x] = v;
-        tb[threadIdx.x] = b;
+        v = wave_max(v);
+        b = __any(b);
+        if ((threadIdx.x & 63) == 0) {
+            tv[threadIdx.x >> 6] = v;
+            tb[threadIdx.x >> 6] = b;
+        }
         __syncthreads();
         if (threadIdx.x == 0) {
             float mv = 0.f;
             int any = 0;
-            for (int i = 0; i < kFinThreads; ++i) {
+#pragma unroll
+            for (int i = 0; i < kFinThreads / 64; ++i) {
                 mv = fmaxf(mv, tv[i]);
                 any |= tb[i];
             }

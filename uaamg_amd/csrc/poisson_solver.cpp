@@ -259,6 +259,16 @@ int PoissonDevice::init(PoissonHierarchyHost&& h, const SolverOptions& opt) {
     return acquire_device();
 }
 
+// Whether level 0's W-cycle visit runs as block-visit launches too (FP32 form;
+// a matter of its size, see kBlock0Leaves).
+bool PoissonDevice::block0() const {
+    if (host_.levels.size() < 2 || opt_.precision != 0 || (opt_.flags & (1 | 16)) || std::getenv("UAAMG_BLOCK_LEAVES"))
+        return false;
+    int64_t most = kBlock0Leaves;
+    if (const char* env = std::getenv("UAAMG_BLOCK0_LEAVES")) most = std::atoll(env);
+    return int64_t(host_.levels[0].nleaf()) <= most;
+}
+
 // Device memory of the hierarchy, the PCG vectors and the scratch: one arena.
 size_t PoissonDevice::device_bytes() const {
     const int L = int(host_.levels.size());
@@ -275,7 +285,7 @@ size_t PoissonDevice::device_bytes() const {
         add(n * sizeof(int64_t));
         add(n * sizeof(int32_t));         // parent
         add(n * 8 * sizeof(int32_t));     // child
-        if (l >= 1) add(n * 27 * kNb27Stride * sizeof(int32_t));   // neighbourhood records
+        if (l >= 1 || block0()) add(n * 27 * kNb27Stride * sizeof(int32_t));   // neighbourhood records
         size_t nslot[kNumCoef] = {0, 0, 0, 0, 0};
         for (int k = 0; k < kNumCoef; ++k)
             for (size_t i = 0; i < n && !hl.keep[k].empty(); ++i) nslot[k] += hl.keep[k][i] ? 1 : 0;
@@ -355,7 +365,7 @@ int PoissonDevice::acquire_device() {
                                   "upload leaf records"))
             return -3;
         std::vector<int32_t> nbrec;
-        if (l >= 1 && lv_[l].v.nb27 && !parent.empty()) {
+        if (lv_[l].v.nb27 && !parent.empty()) {
             const auto& hl = host_.levels[l];
             const size_t n = hl.nleaf();
             std::vector<int32_t> ids(n * 27);
@@ -435,6 +445,7 @@ int PoissonDevice::acquire_device() {
         use_block_.assign(size_t(L), 0);
         for (int l = 1; l + 1 < L; ++l)
             use_block_[size_t(l)] = int64_t(host_.levels[l].nleaf()) <= block_max_leaves_ ? 1 : 0;
+        if (block0()) use_block_[0] = 1;
         tune_pending = block_max_leaves_ > 0 && !fixed;
     }
     if (opt_.precision != 0 && opt_.precision != 1) {
@@ -730,9 +741,9 @@ int PoissonDevice::upload_level(const PoissonLevelHost& h, DevLevel& d, bool spa
     };
     v.mask = static_cast<const uint64_t*>(up(h.mask.data(), n * 8 * sizeof(uint64_t)));
     v.nbr = static_cast<const int32_t*>(up(h.nbr.data(), n * 6 * sizeof(int32_t)));
-    // neighbourhood records of the block-visit kernels (levels >= 1), filled
-    // once the parents are known (acquire_device)
-    v.nb27 = h.level >= 1 ? static_cast<const int32_t*>(arena_.take(std::max<size_t>(n * 27 * kNb27Stride * 4, 4)))
+    // neighbourhood records of the block-visit kernels, filled once the parents
+    // are known (acquire_device)
+    v.nb27 = h.level >= 1 || block0() ? static_cast<const int32_t*>(arena_.take(std::max<size_t>(n * 27 * kNb27Stride * 4, 4)))
                           : nullptr;
     int32_t count[kNumCoef] = {0, 0, 0, 0, 0};
     for (size_t i = 0; i < n; ++i)
@@ -1049,7 +1060,7 @@ void PoissonDevice::precond_fused(int l, float* X, const float* B, bool skip_fir
     const bool weighted = opt_.smoother == kWeightedJacobi;
     auto wpre = [&](int i) { return weighted ? 6.0f / 7.0f : scheduled_weight(kSweeps, i); };
     auto wpost = [&](int i) { return weighted ? 6.0f / 7.0f : scheduled_weight(kSweeps, kSweeps - 1 - i); };
-    if (l >= 1 && l + 1 != tail_level_ && use_block_[size_t(l)]) {
+    if (l + 1 != tail_level_ && use_block_[size_t(l)]) {
         // two launches per visit: pre-smoothing + residual + restriction, then
         // prolongation + post-smoothing (the coarser visits run in between)
         DevLevel& c = lv_[l + 1];
@@ -1058,11 +1069,12 @@ void PoissonDevice::precond_fused(int l, float* X, const float* B, bool skip_fir
             check(launch_block_post_cg(v, cv_, coarsest_dof_of_, c.B, c.X, d.T, B, X, wpost(0), wpost(1), wpost(2),
                                        stream_),
                   "coarsest + block post");
-            return;
+        } else {
+            precond(l + 1, c.X, c.B, true, -1);
+            if (l + 1 != L - 1) precond(l + 1, c.X, c.B, false, -1);
+            check(launch_block_post(v, d.T, c.X, B, X, wpost(0), wpost(1), wpost(2), stream_), "block post");
         }
-        precond(l + 1, c.X, c.B, true, -1);
-        if (l + 1 != L - 1) precond(l + 1, c.X, c.B, false, -1);
-        check(launch_block_post(v, d.T, c.X, B, X, wpost(0), wpost(1), wpost(2), stream_), "block post");
+        if (dot_target >= 0) check(launch_dot(v, X, B, sc_, partials_, dot_target, stream_), "dot");
         return;
     }
     float* cur = X;

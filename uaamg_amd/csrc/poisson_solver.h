@@ -62,6 +62,11 @@ public:
     static constexpr int kSuccess = 0;
     static constexpr int kFailed = 1;
     static constexpr int kMaxReplacements = 4;
+    // Level 0 runs block visits up to this many leaves (each visit two launches
+    // instead of six, its own dot product behind them). Whole solves, block
+    // visits / sweeps on level 0, with 38 leaves: 588 / 701 us, 119: 685 / 770,
+    // 278: 835 / 888, 503: 933 / 981, 774: 1312 / 1303, 1269: 1652 / 1610.
+    static constexpr int64_t kBlock0Leaves = 600;
     static constexpr int kTuneMaxLeaves = 4096;   // coarse levels above this size keep the per-sweep kernels
 
     ~PoissonDevice();
@@ -123,8 +128,9 @@ public:
     // choice came from (ms per visit pair; -1 where the level was not timed).
     const std::vector<uint8_t>& block_levels() const { return use_block_; }
     // the block post-visit of level l also runs the coarsest solve
+    bool block0() const;
     bool post_cg_level(int l) const {
-        return post_cg_ && l >= 1 && l + 2 == nlevels() && size_t(l) < use_block_.size() && use_block_[size_t(l)] &&
+        return post_cg_ && l + 2 == nlevels() && size_t(l) < use_block_.size() && use_block_[size_t(l)] &&
                l + 1 != tail_level_;
     }
     float tune_ms(int level, int variant) const {
