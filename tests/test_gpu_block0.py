@@ -10,7 +10,7 @@ import uaamg_amd as U
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("config,n", [(0, 20), (0, 33), (3, 47), (1, 64), (0, 75)])
+@pytest.mark.parametrize("config,n", [(0, 24), (0, 33), (3, 47), (1, 64), (0, 75)])
 @pytest.mark.parametrize("smoother", [0, 1])
 def test_block_visits_on_level_0(hip_available, monkeypatch, config, n, smoother):
     s = U.Scene(config, n, seed=n)

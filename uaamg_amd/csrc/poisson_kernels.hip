@@ -8,15 +8,16 @@
 #include <cfloat>
 
 #include "stencil_device.h"
+#include "stencil_half.h"
 
 namespace uaamg {
 namespace {
 
 using namespace dev;
 
-template <int MODE, bool kLevel0, class VX = float, class VB = float, class VY = float>
-__global__ __launch_bounds__(kBlockThreads) void apply_kernel(LevelView L, const VX* X, const VB* B, VY* Y, float w,
-                                                              float one_minus_w) {
+template <int MODE, bool kLevel0>
+__global__ __launch_bounds__(kBlockThreads) void apply_kernel(LevelView L, const float* X, const float* B, float* Y,
+                                                              float w, float one_minus_w) {
     const int leaf = wave_leaf();
     if (leaf >= L.nleaf) return;
     const int lane = threadIdx.x & 63;
@@ -25,7 +26,7 @@ __global__ __launch_bounds__(kBlockThreads) void apply_kernel(LevelView L, const
     const uint32_t rm = row_mask(L, leaf, lane);
     const LeafRec R = leaf_rec(L, leaf);
     float xc[8], s[8], y[8];
-    stencil_offdiag(L, R, PlainSrcT<VX>{X}, leaf, lane, xc, s);
+    stencil_offdiag(L, R, PlainSrc{X}, leaf, lane, xc, s);
     const int sd = R.sd;
     const size_t row = size_t(leaf) * 512 + lane * 8;
     if (MODE == kModeRedGS || MODE == kModeBlackGS) {
@@ -57,15 +58,6 @@ __global__ __launch_bounds__(kBlockThreads) void apply_kernel(LevelView L, const
             if (MODE == kModeResidual) {
 #pragma unroll
                 for (int z = 0; z < 8; ++z) y[z] = b[z] - ax[z];
-            } else if (MODE == kModeJacobi) {
-                float inv[8];
-                ld8_slot(L.invdiag, sd, lane, L.dflt_invdiag, inv);
-#pragma unroll
-                for (int z = 0; z < 8; ++z) {
-                    float r = b[z] - ax[z];
-                    r = r * inv[z];
-                    y[z] = fmaf(w, r, xc[z]);
-                }
             } else {   // SPAI0
                 float sp[8];
                 ld8_slot(L.spai0, R.ssp, lane, L.dflt_spai0, sp);
@@ -180,75 +172,85 @@ __global__ __launch_bounds__(kBlockThreads) void prolong_add_kernel(LevelView Fl
     st8(Fv + row, y);
 }
 
-// First two scheduled/weighted Jacobi sweeps from a zero guess in one pass:
+// ---- the Jacobi-family passes, on half rows (stencil_half.h). kLevel0 only
+// names the level in profiles.
+template <class Src, class VB, class VY>
+__device__ __forceinline__ void jacobi_half(const LevelView& L, const Src& src, const VB* B, VY* Y, float w) {
+    __shared__ float tiles[kWavesPerBlock / 2][512];   // a workgroup holds whole leaves
+    HalfPos p = half_pos();
+    const bool valid = p.leaf < L.nleaf;
+    if (!valid) p.leaf = L.nleaf - 1;   // meets the others at the barrier, stores nothing
+    const uint32_t rm = half_row_mask(L, p);
+    const LeafRec R = leaf_rec(L, p.leaf);
+    const size_t at = size_t(p.leaf) * 512 + p.row * 8 + p.z0;
+    float xc[4], s[4], b[4], y[4];
+    typename Src::Quad c;
+    half_offdiag<true>(L, R, src, p, tiles[threadIdx.x >> 7], c, xc, s);
+    ldh(B + at, b);
+    half_jacobi(L, R, p, xc, s, b, w, rm >> p.z0, y);
+    if (valid && rm) sth(Y + at, y);   // rows without a DOF are not written
+}
+
+// One weighted Jacobi sweep. Against full rows (one lane per z-row of eight),
+// at 12193 / 92428 leaves of level 0: 15.7 / 134 us (17.2 / 157), 3.6 / 11.4 us
+// at 282 / 12247 leaves (4.4 / 12.5); bound by HBM and L2 misses.
+template <bool kLevel0, class VX, class VB, class VY>
+__global__ __launch_bounds__(kBlockThreads) void jacobi_half_kernel(LevelView L, const VX* X, const VB* B, VY* Y,
+                                                                    float w) {
+    jacobi_half(L, PlainHalf<VX>{X}, B, Y, w);
+}
+
+// First two scheduled / weighted Jacobi sweeps from a zero guess in one pass:
 // the first sweep's result is rebuilt where the second sweep reads it.
-template <bool kLevel0, class VB = float, class VY = float>
-__global__ __launch_bounds__(kBlockThreads) void jacobi_first2_kernel(LevelView L, const VB* B, VY* Y, float w0,
-                                                                      float w1) {
-    const int leaf = wave_leaf();
-    if (leaf >= L.nleaf) return;
-    const int lane = threadIdx.x & 63;
-    const uint32_t rm = row_mask(L, leaf, lane);
-    const LeafRec R = leaf_rec(L, leaf);
-    const FirstJacobiSrcT<VB> src{B, L.invdiag, L.dflt_invdiag, w0};
-    float xc[8], s[8], y[8];
-    stencil_offdiag(L, R, src, leaf, lane, xc, s);
-    jacobi_row(L, R, leaf, lane, xc, s, B, w1, y);
-    if (rm == 0) return;
-    mask_row(rm, y);
-    st8(Y + size_t(leaf) * 512 + lane * 8, y);
+// 16.3 / 154 us at 12193 / 92428 leaves (full rows 21.5 / 191).
+template <bool kLevel0, class VB, class VY>
+__global__ __launch_bounds__(kBlockThreads) void jacobi_first2_half_kernel(LevelView L, const VB* B, VY* Y, float w0,
+                                                                           float w1) {
+    jacobi_half(L, FirstHalf<VB>{B, L.invdiag, L.dflt_invdiag, w0}, B, Y, w1);
 }
 
 // Prolongation (x += P x_coarse) fused into the first post-smoothing sweep.
-template <bool kLevel0, class V = float, class VB = float>
-__global__ __launch_bounds__(kBlockThreads) void prolong_jacobi_kernel(LevelView L, const V* X, const V* Xc,
-                                                                       const VB* B, V* Y, float w) {
-    const int leaf = wave_leaf();
-    if (leaf >= L.nleaf) return;
-    const int lane = threadIdx.x & 63;
-    const uint32_t rm = row_mask(L, leaf, lane);
-    const LeafRec R = leaf_rec(L, leaf);
-    const ProlongSrcT<V> src{X, Xc, L.mask};
-    float xc[8], s[8], y[8];
-    stencil_offdiag(L, R, src, leaf, lane, xc, s);
-    jacobi_row(L, R, leaf, lane, xc, s, B, w, y);
-    if (rm == 0) return;
-    mask_row(rm, y);
-    st8(Y + size_t(leaf) * 512 + lane * 8, y);
+// 20.5 / 182 us at 12193 / 92428 leaves (full rows 23.4 / 206).
+template <bool kLevel0, class V, class VB>
+__global__ __launch_bounds__(kBlockThreads) void prolong_jacobi_half_kernel(LevelView L, const V* X, const V* Xc,
+                                                                            const VB* B, V* Y, float w) {
+    jacobi_half(L, ProlongHalf<V>{X, Xc, L.mask}, B, Y, w);
 }
 
-// Residual r = b - A x of a fine leaf, restricted in the same pass: each
-// coarse voxel's eight children lie in one fine leaf, so the leaf writes the
-// 4^3 octant of its parent coarse leaf (restriction, :1624-1684, sums the
-// children in x,y,z nested order and scales by 1/8).
-template <bool kLevel0, class V = float, class VB = float>
-__global__ __launch_bounds__(kBlockThreads) void residual_restrict_kernel(LevelView F, const V* X, const VB* B,
-                                                                          V* Cv) {
-    __shared__ float rs[kWavesPerBlock][512];
-    const int wave = threadIdx.x >> 6;
-    const int lane = threadIdx.x & 63;
-    const int leaf = wave_leaf();
-    const bool valid = leaf < F.nleaf;
-    float r[8];
-    fill8(r, 0.f);
+// Residual r = b - A x of half a fine leaf, restricted in the same pass: each
+// coarse voxel's eight children lie in one half, so the wavefront writes its
+// half of the parent coarse leaf's 4^3 octant (restriction, :1624-1684, sums
+// the children in x,y,z nested order and scales by 1/8).
+template <bool kLevel0, class V, class VB>
+__global__ __launch_bounds__(kBlockThreads) void residual_restrict_half_kernel(LevelView F, const V* X, const VB* B,
+                                                                               V* Cv) {
+    __shared__ float rs[kWavesPerBlock][256];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const HalfPos p = half_pos();
+    const bool valid = p.leaf < F.nleaf;
+    float r[4];
+    fillh(r, 0.f);
     int par = -1;
     if (valid) {
-        const uint32_t rm = row_mask(F, leaf, lane);
-        const LeafRec R = leaf_rec(F, leaf);
+        const uint32_t m = half_row_mask(F, p) >> p.z0;
+        const LeafRec R = leaf_rec(F, p.leaf);
         par = R.par;
-        float xc[8], s[8], dg[8], b[8];
-        stencil_offdiag(F, R, PlainSrcT<V>{X}, leaf, lane, xc, s);
-        ld8_slot(F.diag, R.sd, lane, F.dflt_diag, dg);
-        ld8(B + size_t(leaf) * 512 + lane * 8, b);
+        const int off = p.row * 8 + p.z0;
+        float xc[4], s[4], dg[4], b[4];
+        typename PlainHalf<V>::Quad c;
+        half_offdiag<false>(F, R, PlainHalf<V>{X}, p, nullptr, c, xc, s);
+        ldh_slot(F.diag, R.sd, off, F.dflt_diag, dg);
+        ldh(B + size_t(p.leaf) * 512 + off, b);
 #pragma unroll
-        for (int z = 0; z < 8; ++z) r[z] = b[z] - fmaf(xc[z], dg[z], s[z]);
-        mask_row(rm, r);
+        for (int z = 0; z < 4; ++z) {
+            const float v = b[z] - fmaf(xc[z], dg[z], s[z]);
+            r[z] = ((m >> z) & 1u) ? v : 0.f;
+        }
     }
-#pragma unroll
-    for (int z = 0; z < 8; ++z) rs[wave][lane * 8 + z] = r[z];
+    sth(&rs[wave][lane * 4], r);   // row (within the half) * 8 + z
     __syncthreads();
-    if (!valid) return;
-    const int cx = lane >> 4, cy = (lane >> 2) & 3, cz = lane & 3;
+    if (!valid || par < 0 || lane >= 32) return;   // every DOF leaf has a parent; par is a bounds guard
+    const int cx = lane >> 4, cy = (lane >> 2) & 3, cz = lane & 3;   // cx within the half
     float sum = 0.f;
 #pragma unroll
     for (int ii = 0; ii < 2; ++ii)
@@ -256,13 +258,11 @@ __global__ __launch_bounds__(kBlockThreads) void residual_restrict_kernel(LevelV
         for (int jj = 0; jj < 2; ++jj)
 #pragma unroll
             for (int kk = 0; kk < 2; ++kk) sum += rs[wave][((2 * cx + ii) * 8 + (2 * cy + jj)) * 8 + 2 * cz + kk];
-    const int p = par;
-    if (p < 0) return;   // every DOF leaf has a parent; kept as a bounds guard
-    const int cl = p >> 3, oct = p & 7;
-    const int off = ((cx + 4 * ((oct >> 2) & 1)) * 8 + (cy + 4 * ((oct >> 1) & 1))) * 8 + cz + 4 * (oct & 1);
+    const int cl = par >> 3, oct = par & 7;
+    const int off = ((cx + 2 * (p.row >> 5) + 4 * ((oct >> 2) & 1)) * 8 + (cy + 4 * ((oct >> 1) & 1))) * 8 + cz +
+                    4 * (oct & 1);
     st1(Cv + size_t(cl) * 512 + off, sum * 0.125f);
 }
-
 
 __global__ __launch_bounds__(kBlockThreads) void scatter_dof_kernel(LevelView L, const float* dv, float* Y) {
     const int leaf = wave_leaf();
@@ -295,6 +295,47 @@ __global__ __launch_bounds__(kBlockThreads) void gather_dof_kernel(LevelView L, 
 }
 
 
+// level 0 and the coarse levels run the same code under two names
+template <class F0, class F1>
+hipError_t by_level(const LevelView& L, const F0& level0, const F1& coarse) {
+    if (L.nleaf <= 0) return hipSuccess;
+    if (L.level == 0) level0();
+    else coarse();
+    return hipGetLastError();
+}
+
+template <class VX, class VB, class VY>
+hipError_t jacobi_t(const LevelView& L, const VX* x, const VB* b, VY* y, float w, hipStream_t s) {
+    const unsigned g = half_grid(L.nleaf);
+    return by_level(
+        L, [&] { jacobi_half_kernel<true><<<g, kBlockThreads, 0, s>>>(L, x, b, y, w); },
+        [&] { jacobi_half_kernel<false><<<g, kBlockThreads, 0, s>>>(L, x, b, y, w); });
+}
+
+template <class VB, class VY>
+hipError_t jacobi_first2_t(const LevelView& L, const VB* b, VY* y, float w0, float w1, hipStream_t s) {
+    const unsigned g = half_grid(L.nleaf);
+    return by_level(
+        L, [&] { jacobi_first2_half_kernel<true><<<g, kBlockThreads, 0, s>>>(L, b, y, w0, w1); },
+        [&] { jacobi_first2_half_kernel<false><<<g, kBlockThreads, 0, s>>>(L, b, y, w0, w1); });
+}
+
+template <class V, class VB>
+hipError_t prolong_jacobi_t(const LevelView& L, const V* x, const V* xc, const VB* b, V* y, float w, hipStream_t s) {
+    const unsigned g = half_grid(L.nleaf);
+    return by_level(
+        L, [&] { prolong_jacobi_half_kernel<true><<<g, kBlockThreads, 0, s>>>(L, x, xc, b, y, w); },
+        [&] { prolong_jacobi_half_kernel<false><<<g, kBlockThreads, 0, s>>>(L, x, xc, b, y, w); });
+}
+
+template <class V, class VB>
+hipError_t residual_restrict_t(const LevelView& L, const V* x, const VB* b, V* cb, hipStream_t s) {
+    const unsigned g = half_grid(L.nleaf);
+    return by_level(
+        L, [&] { residual_restrict_half_kernel<true><<<g, kBlockThreads, 0, s>>>(L, x, b, cb); },
+        [&] { residual_restrict_half_kernel<false><<<g, kBlockThreads, 0, s>>>(L, x, b, cb); });
+}
+
 }  // namespace
 
 hipError_t launch_apply(const LevelView& L, int mode, const float* x, const float* b, float* y, float w,
@@ -302,11 +343,11 @@ hipError_t launch_apply(const LevelView& L, int mode, const float* x, const floa
     if (L.nleaf <= 0) return hipSuccess;
     const dim3 g(grid_for(L.nleaf)), t(kBlockThreads);
     const float omw = 1.0f - w;
+    if (mode == kModeJacobi) return jacobi_t(L, x, b, y, w, s);
     if (L.level == 0) {
         switch (mode) {
             case kModeLaplacian: apply_kernel<kModeLaplacian, true><<<g, t, 0, s>>>(L, x, b, y, w, omw); break;
             case kModeResidual: apply_kernel<kModeResidual, true><<<g, t, 0, s>>>(L, x, b, y, w, omw); break;
-            case kModeJacobi: apply_kernel<kModeJacobi, true><<<g, t, 0, s>>>(L, x, b, y, w, omw); break;
             case kModeSpai0: apply_kernel<kModeSpai0, true><<<g, t, 0, s>>>(L, x, b, y, w, omw); break;
             case kModeRedGS: apply_kernel<kModeRedGS, true><<<g, t, 0, s>>>(L, x, b, y, w, omw); break;
             case kModeBlackGS: apply_kernel<kModeBlackGS, true><<<g, t, 0, s>>>(L, x, b, y, w, omw); break;
@@ -316,7 +357,6 @@ hipError_t launch_apply(const LevelView& L, int mode, const float* x, const floa
         switch (mode) {
             case kModeLaplacian: apply_kernel<kModeLaplacian, false><<<g, t, 0, s>>>(L, x, b, y, w, omw); break;
             case kModeResidual: apply_kernel<kModeResidual, false><<<g, t, 0, s>>>(L, x, b, y, w, omw); break;
-            case kModeJacobi: apply_kernel<kModeJacobi, false><<<g, t, 0, s>>>(L, x, b, y, w, omw); break;
             case kModeSpai0: apply_kernel<kModeSpai0, false><<<g, t, 0, s>>>(L, x, b, y, w, omw); break;
             case kModeRedGS: apply_kernel<kModeRedGS, false><<<g, t, 0, s>>>(L, x, b, y, w, omw); break;
             case kModeBlackGS: apply_kernel<kModeBlackGS, false><<<g, t, 0, s>>>(L, x, b, y, w, omw); break;
@@ -358,91 +398,56 @@ hipError_t launch_gather_dof(const LevelView& L, const float* bricks, float* dof
 }
 
 hipError_t launch_jacobi_first2(const LevelView& L, const float* b, float* y, float w0, float w1, hipStream_t s) {
-    if (L.nleaf <= 0) return hipSuccess;
-    if (L.level == 0) jacobi_first2_kernel<true><<<grid_for(L.nleaf), kBlockThreads, 0, s>>>(L, b, y, w0, w1);
-    else jacobi_first2_kernel<false><<<grid_for(L.nleaf), kBlockThreads, 0, s>>>(L, b, y, w0, w1);
-    return hipGetLastError();
+    return jacobi_first2_t(L, b, y, w0, w1, s);
 }
 
 hipError_t launch_prolong_jacobi(const LevelView& L, const float* x, const float* xc, const float* b, float* y,
                                  float w, hipStream_t s) {
-    if (L.nleaf <= 0) return hipSuccess;
-    if (L.level == 0) prolong_jacobi_kernel<true><<<grid_for(L.nleaf), kBlockThreads, 0, s>>>(L, x, xc, b, y, w);
-    else prolong_jacobi_kernel<false><<<grid_for(L.nleaf), kBlockThreads, 0, s>>>(L, x, xc, b, y, w);
-    return hipGetLastError();
+    return prolong_jacobi_t(L, x, xc, b, y, w, s);
 }
 
 hipError_t launch_residual_restrict(const LevelView& fine, const float* x, const float* b, float* coarse_b,
                                     hipStream_t s) {
-    if (fine.nleaf <= 0) return hipSuccess;
-    if (fine.level == 0)
-        residual_restrict_kernel<true><<<grid_for(fine.nleaf), kBlockThreads, 0, s>>>(fine, x, b, coarse_b);
-    else residual_restrict_kernel<false><<<grid_for(fine.nleaf), kBlockThreads, 0, s>>>(fine, x, b, coarse_b);
-    return hipGetLastError();
+    return residual_restrict_t(fine, x, b, coarse_b, s);
 }
 
 // ---- mixed-precision W-cycle launchers (level 0 reads the FP32 PCG residual)
 hipError_t launch_jacobi_first2(const LevelView& L, const float* b, bf16* y, float w0, float w1, hipStream_t s) {
-    if (L.nleaf <= 0) return hipSuccess;
-    jacobi_first2_kernel<true, float, bf16><<<grid_for(L.nleaf), kBlockThreads, 0, s>>>(L, b, y, w0, w1);
-    return hipGetLastError();
+    return jacobi_first2_t(L, b, y, w0, w1, s);
 }
-
 hipError_t launch_jacobi_first2(const LevelView& L, const bf16* b, bf16* y, float w0, float w1, hipStream_t s) {
-    if (L.nleaf <= 0) return hipSuccess;
-    jacobi_first2_kernel<false, bf16, bf16><<<grid_for(L.nleaf), kBlockThreads, 0, s>>>(L, b, y, w0, w1);
-    return hipGetLastError();
-}
-
-template <bool kLevel0, class VX, class VB, class VY>
-static hipError_t jacobi_t(const LevelView& L, const VX* x, const VB* b, VY* y, float w, hipStream_t s) {
-    if (L.nleaf <= 0) return hipSuccess;
-    apply_kernel<kModeJacobi, kLevel0, VX, VB, VY>
-        <<<grid_for(L.nleaf), kBlockThreads, 0, s>>>(L, x, b, y, w, 1.0f - w);
-    return hipGetLastError();
+    return jacobi_first2_t(L, b, y, w0, w1, s);
 }
 
 hipError_t launch_jacobi(const LevelView& L, const bf16* x, const float* b, bf16* y, float w, hipStream_t s) {
-    return jacobi_t<true>(L, x, b, y, w, s);
+    return jacobi_t(L, x, b, y, w, s);
 }
 hipError_t launch_jacobi(const LevelView& L, const bf16* x, const float* b, float* y, float w, hipStream_t s) {
-    return jacobi_t<true>(L, x, b, y, w, s);
+    return jacobi_t(L, x, b, y, w, s);
 }
 hipError_t launch_jacobi(const LevelView& L, const float* x, const float* b, bf16* y, float w, hipStream_t s) {
-    return jacobi_t<true>(L, x, b, y, w, s);
+    return jacobi_t(L, x, b, y, w, s);
 }
 hipError_t launch_jacobi(const LevelView& L, const bf16* x, const bf16* b, bf16* y, float w, hipStream_t s) {
-    return jacobi_t<false>(L, x, b, y, w, s);
+    return jacobi_t(L, x, b, y, w, s);
 }
 
 hipError_t launch_residual_restrict(const LevelView& fine, const bf16* x, const float* b, bf16* coarse_b,
                                     hipStream_t s) {
-    if (fine.nleaf <= 0) return hipSuccess;
-    residual_restrict_kernel<true, bf16, float>
-        <<<grid_for(fine.nleaf), kBlockThreads, 0, s>>>(fine, x, b, coarse_b);
-    return hipGetLastError();
+    return residual_restrict_t(fine, x, b, coarse_b, s);
 }
-
 hipError_t launch_residual_restrict(const LevelView& fine, const bf16* x, const bf16* b, bf16* coarse_b,
                                     hipStream_t s) {
-    if (fine.nleaf <= 0) return hipSuccess;
-    residual_restrict_kernel<false, bf16, bf16>
-        <<<grid_for(fine.nleaf), kBlockThreads, 0, s>>>(fine, x, b, coarse_b);
-    return hipGetLastError();
+    return residual_restrict_t(fine, x, b, coarse_b, s);
 }
 
 hipError_t launch_prolong_jacobi(const LevelView& L, const bf16* x, const bf16* xc, const float* b, bf16* y, float w,
                                  hipStream_t s) {
-    if (L.nleaf <= 0) return hipSuccess;
-    prolong_jacobi_kernel<true, bf16, float><<<grid_for(L.nleaf), kBlockThreads, 0, s>>>(L, x, xc, b, y, w);
-    return hipGetLastError();
+    return prolong_jacobi_t(L, x, xc, b, y, w, s);
 }
-
 hipError_t launch_prolong_jacobi(const LevelView& L, const bf16* x, const bf16* xc, const bf16* b, bf16* y, float w,
                                  hipStream_t s) {
-    if (L.nleaf <= 0) return hipSuccess;
-    prolong_jacobi_kernel<false, bf16, bf16><<<grid_for(L.nleaf), kBlockThreads, 0, s>>>(L, x, xc, b, y, w);
-    return hipGetLastError();
+    return prolong_jacobi_t(L, x, xc, b, y, w, s);
 }
 
 }  // namespace uaamg
