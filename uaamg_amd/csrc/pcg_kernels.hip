@@ -14,6 +14,7 @@
 #include "batch_kernels.h"
 #include "coarsest_device.h"
 #include "stencil_device.h"
+#include "stencil_half.h"
 
 namespace uaamg {
 namespace {
@@ -53,113 +54,135 @@ __device__ __forceinline__ void write_partial(double* partials, double v) {
     if (threadIdx.x == 0) partials[logical_block()] = v;
 }
 
-template <int TARGET>
-__global__ __launch_bounds__(kBlockThreads) void dot_kernel(LevelView L, const float* A, const float* Bv,
-                                                            double* partials) {
-    const int leaf = wave_leaf();
-    const int lane = threadIdx.x & 63;
-    double acc = 0;
-    if (leaf < L.nleaf) {
-        const uint32_t rm = row_mask(L, leaf, lane);
-        if (rm) {
-            float a[8], b[8];
-            const size_t row = size_t(leaf) * 512 + lane * 8;
-            ld8(A + row, a);
-            ld8(Bv + row, b);
+// The dot products run on half rows (stencil_half.h), eight wavefronts to the
+// four leaves of a reduction block. Every kernel that forms one of them, alone
+// or with other work, for one problem or a batch, sums the same way: a lane's
+// four products in z order, the wavefront's butterfly, the wavefronts in order.
+constexpr int kDotWaves = 2 * kWavesPerBlock;
+constexpr int kDotThreads = 64 * kDotWaves;
+
+__device__ __forceinline__ void half_dot(const float a[4], const float b[4], uint32_t m, double& acc) {
 #pragma unroll
-            for (int z = 0; z < 8; ++z)
-                if ((rm >> z) & 1u) acc += double(a[z]) * double(b[z]);
-        }
+    for (int z = 0; z < 4; ++z)
+        if ((m >> z) & 1u) acc += double(a[z]) * double(b[z]);
+}
+
+template <int TARGET>
+__global__ __launch_bounds__(kDotThreads) void dot_kernel(LevelView L, const float* A, const float* Bv,
+                                                          double* partials) {
+    const HalfPos p = half_pos<kDotWaves>();
+    double acc = 0;
+    if (p.leaf < L.nleaf) {
+        const uint32_t m = half_row_mask(L, p) >> p.z0;
+        float a[4], b[4];
+        const size_t at = size_t(p.leaf) * 512 + p.row * 8 + p.z0;
+        ldh(A + at, a);
+        ldh(Bv + at, b);
+        half_dot(a, b, m, acc);
     }
-    write_partial(partials, block_sum<kBlockThreads>(acc));
+    write_partial(partials, block_sum<kDotThreads>(acc));
 }
 
 // z = A p and the partials of <p, z>
-__global__ __launch_bounds__(kBlockThreads) void laplacian_dot_kernel(LevelView L, const float* P, float* Z,
-                                                                      double* partials) {
-    const int leaf = wave_leaf();
-    const int lane = threadIdx.x & 63;
+__global__ __launch_bounds__(kDotThreads) void laplacian_dot_kernel(LevelView L, const float* P, float* Z,
+                                                                    double* partials) {
+    const HalfPos p = half_pos<kDotWaves>();
     double acc = 0;
-    if (leaf < L.nleaf) {
-        const uint32_t rm = row_mask(L, leaf, lane);
-        const LeafRec R = leaf_rec(L, leaf);
-        float xc[8], s[8], dg[8], y[8];
-        stencil_offdiag(L, R, PlainSrc{P}, leaf, lane, xc, s);
-        ld8_slot(L.diag, R.sd, lane, L.dflt_diag, dg);
+    if (p.leaf < L.nleaf) {
+        const uint32_t rm = half_row_mask(L, p), m = rm >> p.z0;
+        const LeafRec R = leaf_rec(L, p.leaf);
+        const int off = p.row * 8 + p.z0;
+        PlainHalf<float>::Quad c;
+        float xc[4], s[4], dg[4], y[4];
+        half_offdiag<false>(L, R, PlainHalf<float>{P}, p, nullptr, c, xc, s);
+        ldh_slot(L.diag, R.sd, off, L.dflt_diag, dg);
 #pragma unroll
-        for (int z = 0; z < 8; ++z) {
-            const bool on = (rm >> z) & 1u;
-            y[z] = on ? fmaf(xc[z], dg[z], s[z]) : 0.f;
-            if (on) acc += double(xc[z]) * double(y[z]);
-        }
-        if (rm) st8(Z + size_t(leaf) * 512 + lane * 8, y);
+        for (int z = 0; z < 4; ++z) y[z] = ((m >> z) & 1u) ? fmaf(xc[z], dg[z], s[z]) : 0.f;
+        half_dot(xc, y, m, acc);
+        if (rm) sth(Z + size_t(p.leaf) * 512 + off, y);
     }
-    write_partial(partials, block_sum<kBlockThreads>(acc));
+    write_partial(partials, block_sum<kDotThreads>(acc));
 }
 
 // Last level-0 smoothing sweep of the W-cycle with the partials of <z, r>:
 // z is the sweep's output and r its right-hand side.
 template <class VX = float>
-__global__ __launch_bounds__(kBlockThreads) void jacobi_dot_kernel(LevelView L, const VX* X, const float* B, float* Y,
-                                                                   float w, double* partials) {
-    const int leaf = wave_leaf();
-    const int lane = threadIdx.x & 63;
+__global__ __launch_bounds__(kDotThreads) void jacobi_dot_kernel(LevelView L, const VX* X, const float* B, float* Y,
+                                                                 float w, double* partials) {
+    __shared__ float tiles[kWavesPerBlock][512];
+    HalfPos p = half_pos<kDotWaves>();
+    const bool valid = p.leaf < L.nleaf;
+    if (!valid) p.leaf = L.nleaf - 1;
+    const uint32_t rm = valid ? half_row_mask(L, p) : 0u, m = rm >> p.z0;
+    const LeafRec R = leaf_rec(L, p.leaf);
+    const size_t at = size_t(p.leaf) * 512 + p.row * 8 + p.z0;
+    typename PlainHalf<VX>::Quad c;
+    float xc[4], s[4], y[4], b[4];
+    half_offdiag<true>(L, R, PlainHalf<VX>{X}, p, tiles[threadIdx.x >> 7], c, xc, s);
+    ldh(B + at, b);
+    half_jacobi(L, R, p, xc, s, b, w, m, y);
+    if (rm) sth(Y + at, y);
     double acc = 0;
-    if (leaf < L.nleaf) {
-        const uint32_t rm = row_mask(L, leaf, lane);
-        const LeafRec R = leaf_rec(L, leaf);
-        float xc[8], s[8], y[8], b[8];
-        stencil_offdiag(L, R, PlainSrcT<VX>{X}, leaf, lane, xc, s);
-        jacobi_row(L, R, leaf, lane, xc, s, B, w, y);
-        mask_row(rm, y);
-        if (rm) st8(Y + size_t(leaf) * 512 + lane * 8, y);
-        ld8(B + size_t(leaf) * 512 + lane * 8, b);
+    half_dot(y, b, m, acc);
+    write_partial(partials, block_sum<kDotThreads>(acc));
+}
+
+// x += alpha p; p' = z + beta p; q = A p' of the lane's voxels; p' goes to a
+// second buffer because neighbouring leaves still read p. Called by every
+// thread of the workgroup (kDotThreads, four leaves); `on`: the workgroup's
+// leaves are updated, else only x is. Returns the lane's share of <p', q>.
+__device__ __forceinline__ double update_step(const LevelView& L, const HalfPos& p, bool valid, bool on,
+                                              const float* Z, const float* P, float* Pn, float* X, float* Q,
+                                              float alpha, float beta, float* tile) {
+    const uint32_t rm = valid ? half_row_mask(L, p) : 0u, m = rm >> p.z0;
+    const size_t at = size_t(p.leaf) * 512 + p.row * 8 + p.z0;
+    float x[4], pv[4];
+    ldh(X + at, x);
+    double acc = 0;
+    if (on) {
+        const LeafRec R = leaf_rec(L, p.leaf);
+        UpdateHalf::Quad c;
+        float pc[4], s[4], dg[4], q[4];
+        half_offdiag<true>(L, R, UpdateHalf{Z, P, beta}, p, tile, c, pc, s);
+        ldh_slot(L.diag, R.sd, p.row * 8 + p.z0, L.dflt_diag, dg);
 #pragma unroll
-        for (int z = 0; z < 8; ++z)
-            if ((rm >> z) & 1u) acc += double(y[z]) * double(b[z]);
+        for (int z = 0; z < 4; ++z) {
+            pv[z] = c.p[z];
+            pc[z] = ((m >> z) & 1u) ? pc[z] : 0.f;
+            q[z] = ((m >> z) & 1u) ? fmaf(pc[z], dg[z], s[z]) : 0.f;
+        }
+        half_dot(pc, q, m, acc);
+        if (rm) {
+            sth(Pn + at, pc);
+            sth(Q + at, q);
+        }
+    } else {
+        ldh(P + at, pv);
     }
-    write_partial(partials, block_sum<kBlockThreads>(acc));
+#pragma unroll
+    for (int z = 0; z < 4; ++z) {
+        const float t = alpha * pv[z];
+        x[z] = ((m >> z) & 1u) ? x[z] + t : x[z];
+    }
+    if (rm) sth(X + at, x);
+    return acc;
 }
 
 // One PCG step across the iteration boundary: x += alpha p; p' = z + beta p;
-// q = A p' and the partials of <p', q>. p' goes to a second buffer because
-// neighbouring leaves still read p. At most 128 VGPRs, so four waves per
-// SIMD fit (the default allocation takes 130: three waves).
-__global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(4))) void update_laplacian_dot_kernel(
-    LevelView L, const float* Z, const float* P, float* Pn, float* X, float* Q, const PcgScalars* sc,
-    double* partials) {
-    const int leaf = wave_leaf();
-    const int lane = threadIdx.x & 63;
-    double acc = 0;
-    if (leaf < L.nleaf) {
-        const uint32_t rm = row_mask(L, leaf, lane);
-        const LeafRec R = leaf_rec(L, leaf);
-        const float alpha = sc->alpha, beta = sc->beta;
-        const size_t row = size_t(leaf) * 512 + lane * 8;
-        float x[8], p[8];
-        ld8(X + row, x);
-        ld8(P + row, p);
-        float pc[8], s[8], dg[8], q[8];
-        stencil_offdiag(L, R, UpdateSrc{Z, P, beta}, leaf, lane, pc, s);
-        ld8_slot(L.diag, R.sd, lane, L.dflt_diag, dg);
-        mask_row(rm, pc);
-#pragma unroll
-        for (int z = 0; z < 8; ++z) {
-            const bool on = (rm >> z) & 1u;
-            if (on) {
-                const float t = alpha * p[z];
-                x[z] = x[z] + t;
-            }
-            q[z] = on ? fmaf(pc[z], dg[z], s[z]) : 0.f;
-            if (on) acc += double(pc[z]) * double(q[z]);
-        }
-        if (rm) {
-            st8(X + row, x);
-            st8(Pn + row, pc);
-            st8(Q + row, q);
-        }
-    }
-    write_partial(partials, block_sum<kBlockThreads>(acc));
+// q = A p' and the partials of <p', q>. Six vectors pass through the kernel, so
+// it is bound by HBM; p' is formed once per voxel and shared through LDS. 279 us
+// at 92428 leaves, 37 at 12193, 7.1 at 1679; with full rows and p' formed again
+// at every stencil point 400 / 45 / 9.4, and as two launches (p', then A p')
+// 301 / 38 / 10.3.
+__global__ __launch_bounds__(kDotThreads) void update_laplacian_dot_kernel(LevelView L, const float* Z, const float* P,
+                                                                           float* Pn, float* X, float* Q,
+                                                                           const PcgScalars* sc, double* partials) {
+    __shared__ float tiles[kWavesPerBlock][512];
+    HalfPos p = half_pos<kDotWaves>();
+    const bool valid = p.leaf < L.nleaf;
+    if (!valid) p.leaf = L.nleaf - 1;
+    const double acc = update_step(L, p, valid, true, Z, P, Pn, X, Q, sc->alpha, sc->beta, tiles[threadIdx.x >> 7]);
+    write_partial(partials, block_sum<kDotThreads>(acc));
 }
 
 // running max|r| of one lane; a NaN or Inf sets `bad`
@@ -430,50 +453,22 @@ __device__ __forceinline__ int leaf_problem(const int32_t* leafprob, int leaf) {
     return __builtin_amdgcn_readfirstlane(leafprob[leaf]);
 }
 
-__global__ __launch_bounds__(kBlockThreads) void bupdate_laplacian_dot_kernel(LevelView L, const int32_t* leafprob,
-                                                                              const BatchPcg* st, const float* Z,
-                                                                              const float* P, float* Pn, float* X,
-                                                                              float* Q, double* partials) {
-    const int leaf = wave_leaf();
-    const int lane = threadIdx.x & 63;
+// a reduction block's leaves belong to one problem, so its threads take the
+// same way through the barrier
+__global__ __launch_bounds__(kDotThreads) void bupdate_laplacian_dot_kernel(LevelView L, const int32_t* leafprob,
+                                                                            const BatchPcg* st, const float* Z,
+                                                                            const float* P, float* Pn, float* X,
+                                                                            float* Q, double* partials) {
+    __shared__ float tiles[kWavesPerBlock][512];
+    HalfPos p = half_pos<kDotWaves>();
+    const bool valid = p.leaf < L.nleaf;
+    if (!valid) p.leaf = L.nleaf - 1;
+    const BatchPcg& sp = st[leaf_problem(leafprob, logical_block() * kWavesPerBlock)];
+    const int state = sp.state;
     double acc = 0;
-    if (leaf < L.nleaf) {
-        const uint32_t rm = row_mask(L, leaf, lane);
-        const LeafRec R = leaf_rec(L, leaf);
-        const BatchPcg& sp = st[leaf_problem(leafprob, leaf)];
-        const int state = sp.state;
-        if (state == kBActive || state == kBConverging) {
-            const float alpha = sp.alpha, beta = sp.beta;
-            const size_t row = size_t(leaf) * 512 + lane * 8;
-            float x[8], p[8];
-            ld8(X + row, x);
-            ld8(P + row, p);
-#pragma unroll
-            for (int k = 0; k < 8; ++k)
-                if ((rm >> k) & 1u) {
-                    const float t = alpha * p[k];
-                    x[k] = x[k] + t;
-                }
-            if (rm) st8(X + row, x);
-            if (state == kBActive) {
-                float pc[8], s[8], dg[8], q[8];
-                stencil_offdiag(L, R, UpdateSrc{Z, P, beta}, leaf, lane, pc, s);
-                mask_row(rm, pc);
-                ld8_slot(L.diag, R.sd, lane, L.dflt_diag, dg);
-#pragma unroll
-                for (int z = 0; z < 8; ++z) {
-                    const bool on = (rm >> z) & 1u;
-                    q[z] = on ? fmaf(pc[z], dg[z], s[z]) : 0.f;
-                    if (on) acc += double(pc[z]) * double(q[z]);
-                }
-                if (rm) {
-                    st8(Pn + row, pc);
-                    st8(Q + row, q);
-                }
-            }
-        }
-    }
-    write_partial(partials, block_sum<kBlockThreads>(acc));
+    if (state == kBActive || state == kBConverging)
+        acc = update_step(L, p, valid, state == kBActive, Z, P, Pn, X, Q, sp.alpha, sp.beta, tiles[threadIdx.x >> 7]);
+    write_partial(partials, block_sum<kDotThreads>(acc));
 }
 
 __global__ __launch_bounds__(kBlockThreads) void baxpy_absmax_kernel(LevelView L, const int32_t* leafprob,
@@ -776,7 +771,7 @@ hipError_t launch_replace64_absmax(const LevelView& L, const float* x, const flo
 hipError_t launch_dot(const LevelView& L, const float* a, const float* b, PcgScalars* sc, double* partials,
                       int target, hipStream_t s) {
     const int g = reduction_blocks(L);
-    dot_kernel<0><<<unsigned(g), kBlockThreads, 0, s>>>(L, a, b, partials);
+    dot_kernel<0><<<unsigned(g), kDotThreads, 0, s>>>(L, a, b, partials);
     if (hipError_t e = hipGetLastError()) return e;
     const int op = target == kDotRho ? kFinRho : (target == kDotSigma ? kFinSigma : kFinRhoNew);
     return finalize(op, g, partials, sc, nullptr, s);
@@ -785,7 +780,7 @@ hipError_t launch_dot(const LevelView& L, const float* a, const float* b, PcgSca
 hipError_t launch_laplacian_dot(const LevelView& L, const float* p, float* z, PcgScalars* sc, double* partials,
                                 hipStream_t s) {
     const int g = reduction_blocks(L);
-    laplacian_dot_kernel<<<unsigned(g), kBlockThreads, 0, s>>>(L, p, z, partials);
+    laplacian_dot_kernel<<<unsigned(g), kDotThreads, 0, s>>>(L, p, z, partials);
     if (hipError_t e = hipGetLastError()) return e;
     return finalize(kFinSigma, g, partials, sc, nullptr, s);
 }
@@ -822,7 +817,7 @@ hipError_t launch_update_x(const LevelView& L, const float* p, float* x, const P
 hipError_t launch_jacobi_dot(const LevelView& L, const float* x, const float* b, float* y, float w, PcgScalars* sc,
                              double* partials, int target, hipStream_t s) {
     const int g = reduction_blocks(L);
-    jacobi_dot_kernel<float><<<unsigned(g), kBlockThreads, 0, s>>>(L, x, b, y, w, partials);
+    jacobi_dot_kernel<float><<<unsigned(g), kDotThreads, 0, s>>>(L, x, b, y, w, partials);
     if (hipError_t e = hipGetLastError()) return e;
     return finalize(target == kDotRho ? kFinRho : kFinRhoNew, g, partials, sc, nullptr, s);
 }
@@ -830,7 +825,7 @@ hipError_t launch_jacobi_dot(const LevelView& L, const float* x, const float* b,
 hipError_t launch_jacobi_dot(const LevelView& L, const bf16* x, const float* b, float* y, float w, PcgScalars* sc,
                              double* partials, int target, hipStream_t s) {
     const int g = reduction_blocks(L);
-    jacobi_dot_kernel<bf16><<<unsigned(g), kBlockThreads, 0, s>>>(L, x, b, y, w, partials);
+    jacobi_dot_kernel<bf16><<<unsigned(g), kDotThreads, 0, s>>>(L, x, b, y, w, partials);
     if (hipError_t e = hipGetLastError()) return e;
     return finalize(target == kDotRho ? kFinRho : kFinRhoNew, g, partials, sc, nullptr, s);
 }
@@ -838,7 +833,7 @@ hipError_t launch_jacobi_dot(const LevelView& L, const bf16* x, const float* b, 
 hipError_t launch_update_laplacian_dot(const LevelView& L, const float* z, const float* p, float* p_new, float* x,
                                        float* q, PcgScalars* sc, double* partials, hipStream_t s) {
     const int g = reduction_blocks(L);
-    update_laplacian_dot_kernel<<<unsigned(g), kBlockThreads, 0, s>>>(L, z, p, p_new, x, q, sc, partials);
+    update_laplacian_dot_kernel<<<unsigned(g), kDotThreads, 0, s>>>(L, z, p, p_new, x, q, sc, partials);
     if (hipError_t e = hipGetLastError()) return e;
     return finalize(kFinSigma, g, partials, sc, nullptr, s);
 }
@@ -860,28 +855,28 @@ hipError_t launch_residual64_partials(const LevelView& L, const float* x, const 
 
 hipError_t launch_dot_partials(const LevelView& L, const float* a, const float* b, double* partials, hipStream_t s) {
     if (L.nleaf <= 0) return hipSuccess;
-    dot_kernel<0><<<grid_for(L.nleaf), kBlockThreads, 0, s>>>(L, a, b, partials);
+    dot_kernel<0><<<grid_for(L.nleaf), kDotThreads, 0, s>>>(L, a, b, partials);
     return hipGetLastError();
 }
 
 hipError_t launch_laplacian_dot_partials(const LevelView& L, const float* p, float* q, double* partials,
                                          hipStream_t s) {
     if (L.nleaf <= 0) return hipSuccess;
-    laplacian_dot_kernel<<<grid_for(L.nleaf), kBlockThreads, 0, s>>>(L, p, q, partials);
+    laplacian_dot_kernel<<<grid_for(L.nleaf), kDotThreads, 0, s>>>(L, p, q, partials);
     return hipGetLastError();
 }
 
 hipError_t launch_jacobi_dot_partials(const LevelView& L, const float* x, const float* b, float* y, float w,
                                       double* partials, hipStream_t s) {
     if (L.nleaf <= 0) return hipSuccess;
-    jacobi_dot_kernel<float><<<grid_for(L.nleaf), kBlockThreads, 0, s>>>(L, x, b, y, w, partials);
+    jacobi_dot_kernel<float><<<grid_for(L.nleaf), kDotThreads, 0, s>>>(L, x, b, y, w, partials);
     return hipGetLastError();
 }
 
 hipError_t launch_jacobi_dot_partials(const LevelView& L, const bf16* x, const float* b, float* y, float w,
                                       double* partials, hipStream_t s) {
     if (L.nleaf <= 0) return hipSuccess;
-    jacobi_dot_kernel<bf16><<<grid_for(L.nleaf), kBlockThreads, 0, s>>>(L, x, b, y, w, partials);
+    jacobi_dot_kernel<bf16><<<grid_for(L.nleaf), kDotThreads, 0, s>>>(L, x, b, y, w, partials);
     return hipGetLastError();
 }
 
@@ -889,7 +884,7 @@ hipError_t launch_bupdate_laplacian_dot(const LevelView& L, const int32_t* leafp
                                         const float* z, const float* p, float* p_new, float* x, float* q,
                                         double* partials, hipStream_t s) {
     if (L.nleaf <= 0) return hipSuccess;
-    bupdate_laplacian_dot_kernel<<<grid_for(L.nleaf), kBlockThreads, 0, s>>>(L, leafprob, st, z, p, p_new, x, q,
+    bupdate_laplacian_dot_kernel<<<grid_for(L.nleaf), kDotThreads, 0, s>>>(L, leafprob, st, z, p, p_new, x, q,
                                                                             partials);
     return hipGetLastError();
 }

@@ -194,28 +194,6 @@ struct ProlongSrcT {
 };
 using ProlongSrc = ProlongSrcT<float>;
 
-// p' = z + beta p (levelXPlusAlphaY, simd_vdb_poisson.cpp:2305-2320), both 0 off the DOFs
-struct UpdateSrc {
-    const float* Z;
-    const float* P;
-    float beta;
-    __device__ __forceinline__ void row(int leaf, int, int, int r, float v[8]) const {
-        float z[8], p[8];
-        ld8(Z + size_t(leaf) * 512 + r * 8, z);
-        ld8(P + size_t(leaf) * 512 + r * 8, p);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const float t = beta * p[k];
-            v[k] = z[k] + t;
-        }
-    }
-    __device__ __forceinline__ float at(int leaf, int, int, int r, int z) const {
-        const size_t i = size_t(leaf) * 512 + r * 8 + z;
-        const float t = beta * P[i];
-        return Z[i] + t;
-    }
-};
-
 // The PCG iterate with its pending update, x + alpha p, formed as the update
 // kernels form it (product, then sum; contraction is off), so that values
 // read here equal the ones the deferred update later stores.
