@@ -39,6 +39,8 @@ SOURCES = [
     "vdb_file.cpp",
     "capi_vdb.cpp",
     "rhs_kernels.hip",
+    "leaf_match.cpp",
+    "leaf_match_kernels.hip",
     "rhs_device.cpp",
     "face_update_kernels.hip",
     "face_update.cpp",

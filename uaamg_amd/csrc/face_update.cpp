@@ -1,8 +1,10 @@
 // Host side of the device pressure-gradient update (face_update.h).
 #include "face_update.h"
 
+#include <algorithm>
 #include <vector>
 
+#include "leaf_match.h"
 #include "leaf_topology.h"
 #include "poisson_solver.h"
 
@@ -12,28 +14,12 @@ namespace {
 
 struct DevBuf {
     void* p = nullptr;
-    ~DevBuf() {
+    void release() {
         if (p) (void)hipFree(p);
+        p = nullptr;
     }
+    ~DevBuf() { release(); }
 };
-
-bool build_lookup(int64_t n, const int32_t* org, LeafLookup& lookup, std::string& err, const char* what) {
-    std::vector<Coord> o(static_cast<size_t>(n));
-    for (int64_t i = 0; i < n; ++i) {
-        o[size_t(i)] = {org[3 * i], org[3 * i + 1], org[3 * i + 2]};
-        if ((o[size_t(i)].x | o[size_t(i)].y | o[size_t(i)].z) & 7) {
-            err = std::string(what) + ": leaf origin not a multiple of 8";
-            return false;
-        }
-    }
-    lookup.build(o);
-    for (size_t i = 0; i < o.size(); ++i)
-        if (lookup.find(o[i]) != int32_t(i)) {
-            err = std::string(what) + ": duplicate leaf origins";
-            return false;
-        }
-    return true;
-}
 
 }  // namespace
 
@@ -59,16 +45,15 @@ int apply_pressure_gradient_device(PoissonDevice& d, const float* pressure_dev, 
         return -3;
     };
     const PoissonLevelHost& l0 = d.host().levels[0];
-    LeafLookup dof_lookup;
-    dof_lookup.build(l0.origin);
     // inputs: liquid phi, face weights, solid velocity
     const char* names[3] = {"liquid_phi", "face_weights", "solid_velocity"};
-    LeafLookup in_lookup[3];
+    LeafMatch match;
+    int in_set[3], ch_set[3];
     DevBuf in_buf[3];
     const float* in_dev[3] = {nullptr, nullptr, nullptr};
     for (int g = 0; g < 3; ++g) {
         const FaceGridRef& r = grids[g];
-        if (!build_lookup(r.nleaf, r.origins, in_lookup[g], err, names[g])) return -1;
+        in_set[g] = match.add(r.nleaf, r.origins);
         if (r.nleaf == 0) continue;
         if (values_on_device) {
             in_dev[g] = r.values;
@@ -81,53 +66,93 @@ int apply_pressure_gradient_device(PoissonDevice& d, const float* pressure_dev, 
         in_dev[g] = static_cast<const float*>(in_buf[g].p);
     }
     const LevelView& v0 = d.level_view(0);
+    int64_t most = 0;
+    for (int c = 0; c < 3; ++c) {
+        ch_set[c] = match.add(channels[c].nleaf, channels[c].origins);
+        most = std::max(most, channels[c].nleaf);
+    }
+    static_assert(sizeof(Coord) == 12, "origins are matched as triples of int32");
+    const int dof = match.add(int64_t(l0.nleaf()), l0.nleaf() ? &l0.origin[0].x : nullptr);
+    // the channels' leaf tables and masks in the handle's grow-only buffer (a repeated call allocates nothing)
+    const size_t tab_bytes = (size_t(most) * kGradTab * sizeof(int32_t) + 255) & ~size_t(255);
+    const size_t act_bytes = size_t(most) * 8 * sizeof(uint64_t);
+    char* aux = static_cast<char*>(d.aux(match.bytes() + 3 * (tab_bytes + act_bytes)));
+    if (!aux) return hip_fail(hipErrorOutOfMemory, "device scratch");
+    auto tab_at = [&](int c) { return reinterpret_cast<int32_t*>(aux + match.bytes() + size_t(c) * tab_bytes); };
+    auto act_at = [&](int c) {
+        return reinterpret_cast<uint64_t*>(aux + match.bytes() + 3 * tab_bytes + size_t(c) * act_bytes);
+    };
+    if (hipError_t e = match.build(aux, s)) return hip_fail(e, "leaf match");
+    // refused origins are found before any channel is touched
+    int32_t bad = -1;
+    if (hipError_t e = hipMemcpyAsync(&bad, match.bad(), sizeof(bad), hipMemcpyDeviceToHost, s))
+        return hip_fail(e, "leaf match");
+    if (hipError_t e = hipStreamSynchronize(s)) return hip_fail(e, "leaf match sync");
+    if (bad >= 0) {
+        const char* what = names[0];
+        bool misaligned = false;
+        for (int g = 0; g < 6; ++g) {
+            const int64_t n = g < 3 ? grids[g].nleaf : channels[g - 3].nleaf;
+            what = g < 3 ? names[g] : "velocity channel";
+            if (bad_origins(n, g < 3 ? grids[g].origins : channels[g - 3].origins, &misaligned)) break;
+        }
+        err = std::string(what) + (misaligned ? ": leaf origin not a multiple of 8" : ": duplicate leaf origins");
+        return -1;
+    }
+    DevBuf vel_b, upd_b, refl_b;   // values held on the host: one channel's at a time
+    auto download = [&](int c) -> int {
+        FaceChannelRef& ch = channels[c];
+        const size_t n = size_t(ch.nleaf), vbytes = n * kLeafSize * sizeof(float);
+        if (n == 0) return 0;
+        if (hipError_t e = hipMemcpyAsync(ch.active, act_at(c), n * 8 * sizeof(uint64_t), hipMemcpyDeviceToHost, s))
+            return hip_fail(e, "download active masks");
+        if (values_on_device) return 0;
+        if (hipError_t e = hipMemcpyAsync(ch.values, vel_b.p, vbytes, hipMemcpyDeviceToHost, s))
+            return hip_fail(e, "download velocity");
+        if (ch.update)
+            if (hipError_t e = hipMemcpyAsync(ch.update, upd_b.p, vbytes, hipMemcpyDeviceToHost, s))
+                return hip_fail(e, "download update");
+        if (ch.reflected)
+            if (hipError_t e = hipMemcpyAsync(ch.reflected, refl_b.p, vbytes, hipMemcpyDeviceToHost, s))
+                return hip_fail(e, "download reflected");
+        if (hipError_t e = hipStreamSynchronize(s)) return hip_fail(e, "pressure gradient sync");
+        for (DevBuf* b : {&vel_b, &upd_b, &refl_b}) b->release();
+        return 0;
+    };
     for (int c = 0; c < 3; ++c) {
         FaceChannelRef& ch = channels[c];
-        LeafLookup vl;
-        if (!build_lookup(ch.nleaf, ch.origins, vl, err, "velocity channel")) return -1;
         if (ch.nleaf == 0) continue;
+        int32_t* const tab_d = tab_at(c);
+        uint64_t* const act_d = act_at(c);
         const size_t n = size_t(ch.nleaf);
-        std::vector<int32_t> tab(n * kGradTab);
-        for (size_t i = 0; i < n; ++i) {
-            const Coord o{ch.origins[3 * i], ch.origins[3 * i + 1], ch.origins[3 * i + 2]};
-            Coord lo = o;
-            lo[c] -= 8;
-            int32_t* t = &tab[i * kGradTab];
-            t[kGradPhi] = in_lookup[0].find(o);
-            t[kGradPhiLow] = in_lookup[0].find(lo);
-            t[kGradDof] = dof_lookup.find(o);
-            t[kGradDofLow] = dof_lookup.find(lo);
-            t[kGradW] = in_lookup[1].find(o);
-            t[kGradSolid] = in_lookup[2].find(o);
-        }
         const size_t vbytes = n * kLeafSize * sizeof(float);
-        // the leaf tables and the masks in the handle's grow-only buffer (a repeated call allocates
-        // nothing; the channels take turns, each synchronised before the next)
-        const size_t tab_bytes = (tab.size() * sizeof(int32_t) + 255) & ~size_t(255);
-        char* aux = static_cast<char*>(d.aux(tab_bytes + n * 8 * sizeof(uint64_t)));
-        if (!aux) return hip_fail(hipErrorOutOfMemory, "device scratch");
-        int32_t* tab_d = reinterpret_cast<int32_t*>(aux);
-        uint64_t* act_d = reinterpret_cast<uint64_t*>(aux + tab_bytes);
-        DevBuf vel_d, upd_d, refl_d;
-        if (hipError_t e = hipMemcpyAsync(tab_d, tab.data(), tab.size() * sizeof(int32_t), hipMemcpyHostToDevice, s))
-            return hip_fail(e, "upload tables");
+        const int here[3] = {0, 0, 0}, low[3] = {c == 0 ? -8 : 0, c == 1 ? -8 : 0, c == 2 ? -8 : 0};
+        std::vector<MatchColumn> cols(kGradTab);
+        auto column = [&](int at, int set, const int* o) { cols[size_t(at)] = {set, {o[0], o[1], o[2]}}; };
+        column(kGradPhi, in_set[0], here);
+        column(kGradPhiLow, in_set[0], low);
+        column(kGradDof, dof, here);
+        column(kGradDofLow, dof, low);
+        column(kGradW, in_set[1], here);
+        column(kGradSolid, in_set[2], here);
+        if (hipError_t e = match.query(ch_set[c], cols, tab_d, s)) return hip_fail(e, "leaf match");
         if (hipError_t e = hipMemcpyAsync(act_d, ch.active, n * 8 * sizeof(uint64_t), hipMemcpyHostToDevice, s))
             return hip_fail(e, "upload active masks");
         float* vel = ch.values;
         float* upd = ch.update;
         float* refl = ch.reflected;
         if (!values_on_device) {
-            if (hipError_t e = hipMalloc(&vel_d.p, vbytes)) return hip_fail(e, "hipMalloc");
-            if (hipError_t e = hipMemcpyAsync(vel_d.p, ch.values, vbytes, hipMemcpyHostToDevice, s))
+            if (hipError_t e = hipMalloc(&vel_b.p, vbytes)) return hip_fail(e, "hipMalloc");
+            if (hipError_t e = hipMemcpyAsync(vel_b.p, ch.values, vbytes, hipMemcpyHostToDevice, s))
                 return hip_fail(e, "upload velocity");
-            vel = static_cast<float*>(vel_d.p);
+            vel = static_cast<float*>(vel_b.p);
             if (ch.update) {
-                if (hipError_t e = hipMalloc(&upd_d.p, vbytes)) return hip_fail(e, "hipMalloc");
-                upd = static_cast<float*>(upd_d.p);
+                if (hipError_t e = hipMalloc(&upd_b.p, vbytes)) return hip_fail(e, "hipMalloc");
+                upd = static_cast<float*>(upd_b.p);
             }
             if (ch.reflected) {
-                if (hipError_t e = hipMalloc(&refl_d.p, vbytes)) return hip_fail(e, "hipMalloc");
-                refl = static_cast<float*>(refl_d.p);
+                if (hipError_t e = hipMalloc(&refl_b.p, vbytes)) return hip_fail(e, "hipMalloc");
+                refl = static_cast<float*>(refl_b.p);
             }
         }
         GradArgs a{};
@@ -149,20 +174,14 @@ int apply_pressure_gradient_device(PoissonDevice& d, const float* pressure_dev, 
         a.friction = friction;
         if (hipError_t e = launch_pressure_gradient(ch.nleaf, a, act_d, vel, upd, refl, s))
             return hip_fail(e, "pressure gradient kernel");
-        if (hipError_t e = hipMemcpyAsync(ch.active, act_d, n * 8 * sizeof(uint64_t), hipMemcpyDeviceToHost, s))
-            return hip_fail(e, "download active masks");
-        if (!values_on_device) {
-            if (hipError_t e = hipMemcpyAsync(ch.values, vel, vbytes, hipMemcpyDeviceToHost, s))
-                return hip_fail(e, "download velocity");
-            if (ch.update)
-                if (hipError_t e = hipMemcpyAsync(ch.update, upd, vbytes, hipMemcpyDeviceToHost, s))
-                    return hip_fail(e, "download update");
-            if (ch.reflected)
-                if (hipError_t e = hipMemcpyAsync(ch.reflected, refl, vbytes, hipMemcpyDeviceToHost, s))
-                    return hip_fail(e, "download reflected");
-        }
-        if (hipError_t e = hipStreamSynchronize(s)) return hip_fail(e, "pressure gradient sync");
+        if (!values_on_device)
+            if (int rc = download(c)) return rc;
     }
+    // values on the device: a channel's masks are uploaded beside the kernel of the one before
+    if (values_on_device)
+        for (int c = 0; c < 3; ++c)
+            if (int rc = download(c)) return rc;
+    if (hipError_t e = hipStreamSynchronize(s)) return hip_fail(e, "pressure gradient sync");
     return 0;
 }
 

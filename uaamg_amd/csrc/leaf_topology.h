@@ -64,7 +64,7 @@ inline TreeOrderKey tree_order_key(const Coord& origin) {
 
 inline bool tree_order_less(const Coord& a, const Coord& b) { return tree_order_key(a) < tree_order_key(b); }
 
-inline uint64_t pack_origin(const Coord& o) {
+constexpr uint64_t pack_origin(const Coord& o) {
     // origins are multiples of 8; 21 bits per axis after the shift covers +-2^23 voxels
     const uint64_t m = (uint64_t(1) << 21) - 1;
     return ((uint64_t(uint32_t(o.x >> 3)) & m) << 42) | ((uint64_t(uint32_t(o.y >> 3)) & m) << 21) |

@@ -4,6 +4,7 @@
 #include <mutex>
 #include <vector>
 
+#include "leaf_match.h"
 #include "leaf_topology.h"
 #include "poisson_solver.h"
 
@@ -50,8 +51,8 @@ struct DevBuf {
     }
 };
 
-// tab_scratch: device memory for the leaf tables (at least kRhsNoAllocMaxLeaves
-// leaves' worth), or null to allocate them for the call
+// tab_scratch: device memory for leaf tables matched on the host (at least
+// kRhsNoAllocMaxLeaves leaves' worth), or null to match them on the device
 int build_rhs_impl(PoissonDevice& d, const RhsGridRef* grids, float* rhs_dof, int32_t* tab_scratch,
                    std::string& err) {
     if (!d.on_device()) {
@@ -76,29 +77,32 @@ int build_rhs_impl(PoissonDevice& d, const RhsGridRef* grids, float* rhs_dof, in
     };
     RhsArgs a{};
     a.invdx = 1.0f / l0.dx;
-    DevBuf vals[kRhsGrids], tab;
-    std::vector<int32_t> table(n0 * kRhsGrids * 4, -1);
+    DevBuf vals[kRhsGrids];
+    auto refusal = [&](bool misaligned) {
+        err = misaligned ? "grid leaf origin not a multiple of 8" : "grid has duplicate leaf origins";
+        return -1;
+    };
+    std::vector<int32_t> table;   // matched on the host
+    LeafMatch match;              // matched on the device
+    int set[kRhsGrids];
+    if (tab_scratch) table.assign(n0 * kRhsGrids * 4, -1);
     for (int g = 0; g < kRhsGrids; ++g) {
         const RhsGridRef& r = grids[g];
-        std::vector<Coord> org(size_t(r.nleaf));
-        for (int64_t i = 0; i < r.nleaf; ++i) {
-            org[size_t(i)] = {r.origins[3 * i], r.origins[3 * i + 1], r.origins[3 * i + 2]};
-            if ((org[size_t(i)].x | org[size_t(i)].y | org[size_t(i)].z) & 7) {
-                err = "grid leaf origin not a multiple of 8";
-                return -1;
+        if (tab_scratch) {
+            bool misaligned;
+            if (bad_origins(r.nleaf, r.origins, &misaligned)) return refusal(misaligned);
+            std::vector<Coord> org(size_t(r.nleaf));
+            for (size_t i = 0; i < org.size(); ++i)
+                org[i] = {r.origins[3 * i], r.origins[3 * i + 1], r.origins[3 * i + 2]};
+            LeafLookup lookup;
+            lookup.build(org);
+            for (size_t i = 0; i < n0; ++i) {
+                const Coord o = l0.origin[i];
+                const Coord at[4] = {o, {o.x + 8, o.y, o.z}, {o.x, o.y + 8, o.z}, {o.x, o.y, o.z + 8}};
+                for (int k = 0; k < 4; ++k) table[(i * kRhsGrids + size_t(g)) * 4 + size_t(k)] = lookup.find(at[k]);
             }
-        }
-        LeafLookup lookup;
-        lookup.build(org);
-        for (size_t i = 0; i < org.size(); ++i)
-            if (lookup.find(org[i]) != int32_t(i)) {
-                err = "grid has duplicate leaf origins";
-                return -1;
-            }
-        for (size_t i = 0; i < n0; ++i) {
-            const Coord o = l0.origin[i];
-            const Coord at[4] = {o, {o.x + 8, o.y, o.z}, {o.x, o.y + 8, o.z}, {o.x, o.y, o.z + 8}};
-            for (int k = 0; k < 4; ++k) table[(i * kRhsGrids + size_t(g)) * 4 + size_t(k)] = lookup.find(at[k]);
+        } else {
+            set[g] = match.add(r.nleaf, r.origins);
         }
         a.g[g].ncomp = r.ncomp;
         for (int c = 0; c < 3; ++c) a.g[g].bg[c] = r.bg[c];
@@ -114,17 +118,39 @@ int build_rhs_impl(PoissonDevice& d, const RhsGridRef* grids, float* rhs_dof, in
             a.g[g].values = static_cast<const float*>(vals[g].p);
         }
     }
-    if (n0 == 0) return 0;
-    void* tab_dev = tab_scratch;
-    if (!tab_dev) {
-        if (hipError_t e = hipMalloc(&tab.p, table.size() * sizeof(int32_t))) return hip_fail(e, "hipMalloc");
-        tab_dev = tab.p;
+    if (tab_scratch) {
+        if (n0 == 0) return 0;
+        if (hipError_t e = hipMemcpyAsync(tab_scratch, table.data(), table.size() * sizeof(int32_t),
+                                          hipMemcpyHostToDevice, s))
+            return hip_fail(e, "upload leaf tables");
+        a.tab = tab_scratch;
+    } else {
+        static_assert(sizeof(Coord) == 12, "origins are matched as triples of int32");
+        const int dof = match.add(int64_t(n0), n0 ? &l0.origin[0].x : nullptr);
+        // in the handle's grow-only buffer: a repeated call allocates nothing
+        char* mem = static_cast<char*>(d.aux(match.bytes() + n0 * kRhsGrids * 4 * sizeof(int32_t)));
+        if (!mem) return hip_fail(hipErrorOutOfMemory, "device scratch");
+        if (hipError_t e = match.build(mem, s)) return hip_fail(e, "leaf match");
+        std::vector<MatchColumn> cols;
+        for (int g = 0; g < kRhsGrids; ++g)
+            for (int k = 0; k < 4; ++k) cols.push_back({set[g], {8 * (k == 1), 8 * (k == 2), 8 * (k == 3)}});
+        int32_t* tab = reinterpret_cast<int32_t*>(mem + match.bytes());
+        if (hipError_t e = match.query(dof, cols, tab, s)) return hip_fail(e, "leaf match");
+        a.tab = tab;
+        a.bad = match.bad();
     }
-    if (hipError_t e = hipMemcpyAsync(tab_dev, table.data(), table.size() * sizeof(int32_t), hipMemcpyHostToDevice, s))
-        return hip_fail(e, "upload leaf tables");
-    a.tab = static_cast<const int32_t*>(tab_dev);
+    int32_t bad = -1;
     if (hipError_t e = launch_poisson_rhs(d.level_view(0), a, rhs_dof, s)) return hip_fail(e, "rhs kernel");
+    if (a.bad)
+        if (hipError_t e = hipMemcpyAsync(&bad, a.bad, sizeof(bad), hipMemcpyDeviceToHost, s))
+            return hip_fail(e, "leaf match");
     if (hipError_t e = hipStreamSynchronize(s)) return hip_fail(e, "rhs sync");
+    if (bad >= 0) {
+        bool misaligned = false;
+        for (int g = 0; g < kRhsGrids; ++g)
+            if (bad_origins(grids[g].nleaf, grids[g].origins, &misaligned)) break;
+        return refusal(misaligned);
+    }
     return 0;
 }
 

@@ -11,48 +11,56 @@ __device__ __forceinline__ float grid_value(const RhsGridDev& g, int32_t leaf, i
     return leaf >= 0 ? g.values[(size_t(leaf) * 512 + off) * size_t(g.ncomp) + comp] : g.bg[comp];
 }
 
-// one wavefront per level-0 DOF leaf, one lane per z-row (the term order of
-// BuildPoissonRhs::operator(), simd_vdb_poisson.cpp:43-84)
+// One wavefront per x-plane of a level-0 DOF leaf, a lane per voxel (the term
+// order of BuildPoissonRhs::operator(), simd_vdb_poisson.cpp:43-84). Bound by
+// HBM: 75 us at 12193 leaves; a lane per z-row, whose voxels lie 32 and 96
+// bytes from the next lane's, took 320.
 __global__ __launch_bounds__(kBlockThreads) void poisson_rhs_kernel(LevelView L, RhsArgs a, float* out) {
-    const int leaf = wave_leaf();
+    const int gw = __builtin_amdgcn_readfirstlane(logical_block() * kWavesPerBlock + int(threadIdx.x >> 6));
+    const int leaf = gw >> 3, lx = gw & 7;
     if (leaf >= L.nleaf) return;
-    const int lane = threadIdx.x & 63;
-    const int lx = lane >> 3, ly = lane & 7;
-    const uint32_t rm = row_mask(L, leaf, lane);
-    if (!rm) return;
+    if (a.bad && *a.bad >= 0) return;
+    const int lane = threadIdx.x & 63, ly = lane >> 3, lz = lane & 7;
+    const uint64_t* mask = L.mask + size_t(leaf) * 8;
+    const uint64_t word = mask[lx];
+    if (!((word >> lane) & 1u)) return;
     const int32_t* t = a.tab + size_t(leaf) * (kRhsGrids * 4);
-    int64_t k = row_dof_base(L, leaf, lane);
-    for (int z = 0; z < 8; ++z) {
-        if (!((rm >> z) & 1u)) continue;
-        float rhs = 0.f;
-        bool nonzero_weight = false;
-        for (int f = 0; f < 6; ++f) {
-            const int ch = f >> 1;
-            const bool positive = (f & 1) == 0;
-            int X = lx + (positive && ch == 0), Y = ly + (positive && ch == 1), Z = z + (positive && ch == 2);
-            int nb = 0;   // 0 own leaf, 1..3 the +x / +y / +z neighbour
-            if (X == 8) { nb = 1; X = 0; }
-            if (Y == 8) { nb = 2; Y = 0; }
-            if (Z == 8) { nb = 3; Z = 0; }
-            const int off = (X << 6) | (Y << 3) | Z;
-            const float weight = grid_value(a.g[kRhsWeight], t[kRhsWeight * 4 + nb], off, ch);
-            if (weight != 0.f) nonzero_weight = true;
-            const float v = grid_value(a.g[kRhsVx + ch], t[(kRhsVx + ch) * 4 + nb], off, 0);
-            const float sv = grid_value(a.g[kRhsSolid], t[kRhsSolid * 4 + nb], off, ch);
-            const float flux = a.invdx * (weight * v + (1.0f - weight) * sv);
-            if (positive) rhs -= flux;
-            else rhs += flux;
-        }
-        if (!nonzero_weight) rhs = 0.f;
-        out[k++] = rhs;
+    // weight, velocity and solid velocity of the faces x+, x-, y+, y-, z+, z-
+    float w[6], v[6], sv[6];
+#pragma unroll
+    for (int f = 0; f < 6; ++f) {
+        const int ch = f >> 1;
+        const bool positive = (f & 1) == 0;
+        const int X = lx + (positive && ch == 0), Y = ly + (positive && ch == 1), Z = lz + (positive && ch == 2);
+        // 0 own leaf, 1..3 the +x / +y / +z neighbour
+        const bool past = positive && (ch == 0 ? X : (ch == 1 ? Y : Z)) == 8;
+        const int nb = past ? 1 + ch : 0;
+        const int off = ((X & 7) << 6) | ((Y & 7) << 3) | (Z & 7);
+        w[f] = grid_value(a.g[kRhsWeight], t[kRhsWeight * 4 + nb], off, ch);
+        v[f] = grid_value(a.g[kRhsVx + ch], t[(kRhsVx + ch) * 4 + nb], off, 0);
+        sv[f] = grid_value(a.g[kRhsSolid], t[kRhsSolid * 4 + nb], off, ch);
     }
+    float rhs = 0.f;
+    bool nonzero_weight = false;
+#pragma unroll
+    for (int f = 0; f < 6; ++f) {
+        if (w[f] != 0.f) nonzero_weight = true;
+        const float flux = a.invdx * (w[f] * v[f] + (1.0f - w[f]) * sv[f]);
+        if ((f & 1) == 0) rhs -= flux;
+        else rhs += flux;
+    }
+    if (!nonzero_weight) rhs = 0.f;
+    int64_t k = L.dofbase[leaf];
+    for (int i = 0; i < lx; ++i) k += __popcll(mask[i]);
+    out[k + __popcll(word & ((uint64_t(1) << lane) - 1))] = rhs;
 }
 
 }  // namespace
 
 hipError_t launch_poisson_rhs(const LevelView& L0, const RhsArgs& a, float* rhs_dof, hipStream_t s) {
     if (L0.nleaf <= 0) return hipSuccess;
-    poisson_rhs_kernel<<<grid_for(L0.nleaf), kBlockThreads, 0, s>>>(L0, a, rhs_dof);
+    static_assert(8 % kWavesPerBlock == 0, "whole blocks of a leaf's planes");
+    poisson_rhs_kernel<<<unsigned(L0.nleaf) * (8 / kWavesPerBlock), kBlockThreads, 0, s>>>(L0, a, rhs_dof);
     return hipGetLastError();
 }
 
