@@ -94,7 +94,7 @@ __global__ __launch_bounds__(kDotThreads) void laplacian_dot_kernel(LevelView L,
         const int off = p.row * 8 + p.z0;
         PlainHalf<float>::Quad c;
         float xc[4], s[4], dg[4], y[4];
-        half_offdiag<false>(L, R, PlainHalf<float>{P}, p, nullptr, c, xc, s);
+        half_offdiag<0>(L, R, PlainHalf<float>{P}, p, nullptr, c, xc, s);
         ldh_slot(L.diag, R.sd, off, L.dflt_diag, dg);
 #pragma unroll
         for (int z = 0; z < 4; ++z) y[z] = ((m >> z) & 1u) ? fmaf(xc[z], dg[z], s[z]) : 0.f;
@@ -117,13 +117,14 @@ __global__ __launch_bounds__(kDotThreads) void jacobi_dot_kernel(LevelView L, co
     const LeafRec R = leaf_rec(L, p.leaf);
     const size_t at = size_t(p.leaf) * 512 + p.row * 8 + p.z0;
     typename PlainHalf<VX>::Quad c;
-    float xc[4], s[4], y[4], b[4];
-    half_offdiag<true>(L, R, PlainHalf<VX>{X}, p, tiles[threadIdx.x >> 7], c, xc, s);
-    ldh(B + at, b);
-    half_jacobi(L, R, p, xc, s, b, w, m, y);
+    JacobiHalf j;
+    float xc[4], s[4], y[4];
+    half_offdiag<kWavesPerBlock>(L, R, PlainHalf<VX>{X}, p, tiles, c, xc, s);
+    j.load(L, R, p, B);
+    j.sweep(xc, s, w, m, y);
     if (rm) sth(Y + at, y);
     double acc = 0;
-    half_dot(y, b, m, acc);
+    half_dot(y, j.b, m, acc);
     write_partial(partials, block_sum<kDotThreads>(acc));
 }
 
@@ -133,7 +134,7 @@ __global__ __launch_bounds__(kDotThreads) void jacobi_dot_kernel(LevelView L, co
 // leaves are updated, else only x is. Returns the lane's share of <p', q>.
 __device__ __forceinline__ double update_step(const LevelView& L, const HalfPos& p, bool valid, bool on,
                                               const float* Z, const float* P, float* Pn, float* X, float* Q,
-                                              float alpha, float beta, float* tile) {
+                                              float alpha, float beta, float (*tiles)[512]) {
     const uint32_t rm = valid ? half_row_mask(L, p) : 0u, m = rm >> p.z0;
     const size_t at = size_t(p.leaf) * 512 + p.row * 8 + p.z0;
     float x[4], pv[4];
@@ -143,8 +144,8 @@ __device__ __forceinline__ double update_step(const LevelView& L, const HalfPos&
         const LeafRec R = leaf_rec(L, p.leaf);
         UpdateHalf::Quad c;
         float pc[4], s[4], dg[4], q[4];
-        half_offdiag<true>(L, R, UpdateHalf{Z, P, beta}, p, tile, c, pc, s);
         ldh_slot(L.diag, R.sd, p.row * 8 + p.z0, L.dflt_diag, dg);
+        half_offdiag<kWavesPerBlock>(L, R, UpdateHalf{Z, P, beta}, p, tiles, c, pc, s);
 #pragma unroll
         for (int z = 0; z < 4; ++z) {
             pv[z] = c.p[z];
@@ -170,8 +171,8 @@ __device__ __forceinline__ double update_step(const LevelView& L, const HalfPos&
 
 // One PCG step across the iteration boundary: x += alpha p; p' = z + beta p;
 // q = A p' and the partials of <p', q>. Six vectors pass through the kernel, so
-// it is bound by HBM; p' is formed once per voxel and shared through LDS. 279 us
-// at 92428 leaves, 37 at 12193, 7.1 at 1679; with full rows and p' formed again
+// it is bound by HBM; p' is formed once per voxel and shared through LDS. 258 us
+// at 92428 leaves, 35 at 12193, 6.8 at 1679; with full rows and p' formed again
 // at every stencil point 400 / 45 / 9.4, and as two launches (p', then A p')
 // 301 / 38 / 10.3.
 __global__ __launch_bounds__(kDotThreads) void update_laplacian_dot_kernel(LevelView L, const float* Z, const float* P,
@@ -181,7 +182,7 @@ __global__ __launch_bounds__(kDotThreads) void update_laplacian_dot_kernel(Level
     HalfPos p = half_pos<kDotWaves>();
     const bool valid = p.leaf < L.nleaf;
     if (!valid) p.leaf = L.nleaf - 1;
-    const double acc = update_step(L, p, valid, true, Z, P, Pn, X, Q, sc->alpha, sc->beta, tiles[threadIdx.x >> 7]);
+    const double acc = update_step(L, p, valid, true, Z, P, Pn, X, Q, sc->alpha, sc->beta, tiles);
     write_partial(partials, block_sum<kDotThreads>(acc));
 }
 
@@ -467,7 +468,7 @@ __global__ __launch_bounds__(kDotThreads) void bupdate_laplacian_dot_kernel(Leve
     const int state = sp.state;
     double acc = 0;
     if (state == kBActive || state == kBConverging)
-        acc = update_step(L, p, valid, state == kBActive, Z, P, Pn, X, Q, sp.alpha, sp.beta, tiles[threadIdx.x >> 7]);
+        acc = update_step(L, p, valid, state == kBActive, Z, P, Pn, X, Q, sp.alpha, sp.beta, tiles);
     write_partial(partials, block_sum<kDotThreads>(acc));
 }
 

@@ -174,47 +174,55 @@ __global__ __launch_bounds__(kBlockThreads) void prolong_add_kernel(LevelView Fl
 
 // ---- the Jacobi-family passes, on half rows (stencil_half.h). kLevel0 only
 // names the level in profiles.
-template <class Src, class VB, class VY>
+// Leaves a workgroup. With 2 / 4 / 8 the sweep takes 132 / 133 / 137 us at 92428
+// leaves, the one after the prolongation 180 / 202 / 254: the more wavefronts
+// meet at the barrier, the fewer hide each other's loads.
+constexpr int kSweepLeaves = 2;
+constexpr int kSweepThreads = 128 * kSweepLeaves;
+
+// kEarly: the sweep's own operands are loaded before the barrier (JacobiHalf)
+template <bool kEarly, class Src, class VB, class VY>
 __device__ __forceinline__ void jacobi_half(const LevelView& L, const Src& src, const VB* B, VY* Y, float w) {
-    __shared__ float tiles[kWavesPerBlock / 2][512];   // a workgroup holds whole leaves
-    HalfPos p = half_pos();
+    __shared__ float tiles[kSweepLeaves][512];   // a workgroup holds whole leaves
+    HalfPos p = half_pos<2 * kSweepLeaves>();
     const bool valid = p.leaf < L.nleaf;
     if (!valid) p.leaf = L.nleaf - 1;   // meets the others at the barrier, stores nothing
     const uint32_t rm = half_row_mask(L, p);
     const LeafRec R = leaf_rec(L, p.leaf);
-    const size_t at = size_t(p.leaf) * 512 + p.row * 8 + p.z0;
-    float xc[4], s[4], b[4], y[4];
+    JacobiHalf j;
+    if (kEarly) j.load(L, R, p, B);
+    float xc[4], s[4], y[4];
     typename Src::Quad c;
-    half_offdiag<true>(L, R, src, p, tiles[threadIdx.x >> 7], c, xc, s);
-    ldh(B + at, b);
-    half_jacobi(L, R, p, xc, s, b, w, rm >> p.z0, y);
-    if (valid && rm) sth(Y + at, y);   // rows without a DOF are not written
+    half_offdiag<kSweepLeaves>(L, R, src, p, tiles, c, xc, s);
+    if (!kEarly) j.load(L, R, p, B);
+    j.sweep(xc, s, w, rm >> p.z0, y);
+    if (valid && rm) sth(Y + size_t(p.leaf) * 512 + p.row * 8 + p.z0, y);   // rows without a DOF are not written
 }
 
 // One weighted Jacobi sweep. Against full rows (one lane per z-row of eight),
-// at 12193 / 92428 leaves of level 0: 15.7 / 134 us (17.2 / 157), 3.6 / 11.4 us
-// at 282 / 12247 leaves (4.4 / 12.5); bound by HBM and L2 misses.
+// at 12193 / 92428 leaves of level 0: 16.0 / 132 us (17.2 / 157), 3.6 / 11.6 us
+// at 282 / 12247 leaves (4.4 / 12.5); at 92428 leaves 0.74 GB pass through HBM, 5.6 TB/s.
 template <bool kLevel0, class VX, class VB, class VY>
-__global__ __launch_bounds__(kBlockThreads) void jacobi_half_kernel(LevelView L, const VX* X, const VB* B, VY* Y,
+__global__ __launch_bounds__(kSweepThreads) void jacobi_half_kernel(LevelView L, const VX* X, const VB* B, VY* Y,
                                                                     float w) {
-    jacobi_half(L, PlainHalf<VX>{X}, B, Y, w);
+    jacobi_half<false>(L, PlainHalf<VX>{X}, B, Y, w);
 }
 
 // First two scheduled / weighted Jacobi sweeps from a zero guess in one pass:
 // the first sweep's result is rebuilt where the second sweep reads it.
-// 16.3 / 154 us at 12193 / 92428 leaves (full rows 21.5 / 191).
+// 16.4 / 143 us at 12193 / 92428 leaves (full rows 21.5 / 191).
 template <bool kLevel0, class VB, class VY>
-__global__ __launch_bounds__(kBlockThreads) void jacobi_first2_half_kernel(LevelView L, const VB* B, VY* Y, float w0,
+__global__ __launch_bounds__(kSweepThreads) void jacobi_first2_half_kernel(LevelView L, const VB* B, VY* Y, float w0,
                                                                            float w1) {
-    jacobi_half(L, FirstHalf<VB>{B, L.invdiag, L.dflt_invdiag, w0}, B, Y, w1);
+    jacobi_half<true>(L, FirstHalf<VB>{B, L.invdiag, L.dflt_invdiag, w0}, B, Y, w1);
 }
 
 // Prolongation (x += P x_coarse) fused into the first post-smoothing sweep.
-// 20.5 / 182 us at 12193 / 92428 leaves (full rows 23.4 / 206).
+// 20.7 / 181 us at 12193 / 92428 leaves (full rows 23.4 / 206).
 template <bool kLevel0, class V, class VB>
-__global__ __launch_bounds__(kBlockThreads) void prolong_jacobi_half_kernel(LevelView L, const V* X, const V* Xc,
+__global__ __launch_bounds__(kSweepThreads) void prolong_jacobi_half_kernel(LevelView L, const V* X, const V* Xc,
                                                                             const VB* B, V* Y, float w) {
-    jacobi_half(L, ProlongHalf<V>{X, Xc, L.mask}, B, Y, w);
+    jacobi_half<false>(L, ProlongHalf<V>{X, Xc, L.mask}, B, Y, w);
 }
 
 // Residual r = b - A x of half a fine leaf, restricted in the same pass: each
@@ -238,7 +246,7 @@ __global__ __launch_bounds__(kBlockThreads) void residual_restrict_half_kernel(L
         const int off = p.row * 8 + p.z0;
         float xc[4], s[4], dg[4], b[4];
         typename PlainHalf<V>::Quad c;
-        half_offdiag<false>(F, R, PlainHalf<V>{X}, p, nullptr, c, xc, s);
+        half_offdiag<0>(F, R, PlainHalf<V>{X}, p, nullptr, c, xc, s);
         ldh_slot(F.diag, R.sd, off, F.dflt_diag, dg);
         ldh(B + size_t(p.leaf) * 512 + off, b);
 #pragma unroll
@@ -306,26 +314,26 @@ hipError_t by_level(const LevelView& L, const F0& level0, const F1& coarse) {
 
 template <class VX, class VB, class VY>
 hipError_t jacobi_t(const LevelView& L, const VX* x, const VB* b, VY* y, float w, hipStream_t s) {
-    const unsigned g = half_grid(L.nleaf);
+    const unsigned g = half_grid(L.nleaf, 2 * kSweepLeaves);
     return by_level(
-        L, [&] { jacobi_half_kernel<true><<<g, kBlockThreads, 0, s>>>(L, x, b, y, w); },
-        [&] { jacobi_half_kernel<false><<<g, kBlockThreads, 0, s>>>(L, x, b, y, w); });
+        L, [&] { jacobi_half_kernel<true><<<g, kSweepThreads, 0, s>>>(L, x, b, y, w); },
+        [&] { jacobi_half_kernel<false><<<g, kSweepThreads, 0, s>>>(L, x, b, y, w); });
 }
 
 template <class VB, class VY>
 hipError_t jacobi_first2_t(const LevelView& L, const VB* b, VY* y, float w0, float w1, hipStream_t s) {
-    const unsigned g = half_grid(L.nleaf);
+    const unsigned g = half_grid(L.nleaf, 2 * kSweepLeaves);
     return by_level(
-        L, [&] { jacobi_first2_half_kernel<true><<<g, kBlockThreads, 0, s>>>(L, b, y, w0, w1); },
-        [&] { jacobi_first2_half_kernel<false><<<g, kBlockThreads, 0, s>>>(L, b, y, w0, w1); });
+        L, [&] { jacobi_first2_half_kernel<true><<<g, kSweepThreads, 0, s>>>(L, b, y, w0, w1); },
+        [&] { jacobi_first2_half_kernel<false><<<g, kSweepThreads, 0, s>>>(L, b, y, w0, w1); });
 }
 
 template <class V, class VB>
 hipError_t prolong_jacobi_t(const LevelView& L, const V* x, const V* xc, const VB* b, V* y, float w, hipStream_t s) {
-    const unsigned g = half_grid(L.nleaf);
+    const unsigned g = half_grid(L.nleaf, 2 * kSweepLeaves);
     return by_level(
-        L, [&] { prolong_jacobi_half_kernel<true><<<g, kBlockThreads, 0, s>>>(L, x, xc, b, y, w); },
-        [&] { prolong_jacobi_half_kernel<false><<<g, kBlockThreads, 0, s>>>(L, x, xc, b, y, w); });
+        L, [&] { prolong_jacobi_half_kernel<true><<<g, kSweepThreads, 0, s>>>(L, x, xc, b, y, w); },
+        [&] { prolong_jacobi_half_kernel<false><<<g, kSweepThreads, 0, s>>>(L, x, xc, b, y, w); });
 }
 
 template <class V, class VB>

@@ -27,7 +27,9 @@ __device__ __forceinline__ HalfPos half_pos() {
     p.z0 = (lane & 1) * 4;
     return p;
 }
-inline unsigned half_grid(int32_t nleaf) { return unsigned((2 * int64_t(nleaf) + kWavesPerBlock - 1) / kWavesPerBlock); }
+inline unsigned half_grid(int32_t nleaf, int waves = kWavesPerBlock) {
+    return unsigned((2 * int64_t(nleaf) + waves - 1) / waves);
+}
 
 // v of the other lane of the pair
 __device__ __forceinline__ float pair_swap(float v) {
@@ -192,14 +194,13 @@ struct UpdateHalf {
 
 // Own operands c and values xc of the source and the off-diagonal sum of the
 // stencil for the lane's four voxels (every lane of the wavefront must be
-// active). With kTile
-// the values of rows inside the leaf come from `tile` (the leaf's 512 values in
-// LDS, formed once by the two wavefronts of the leaf, which share a workgroup)
-// and only rows beyond a face are loaded: for sources of several operands the
-// loads saved are worth the barrier. Every thread of the workgroup must call it.
-template <bool kTile, class Src>
+// active). With kTiles leaves a workgroup (0: none shared) the values inside
+// the leaf come from LDS, where its two wavefronts put them once, and so does
+// the value past a row's end where the workgroup holds the z-neighbour, one
+// brick line a lane otherwise; only rows beyond the x and y faces are loaded. Every thread of the workgroup must call it.
+template <int kTiles, class Src>
 __device__ __forceinline__ void half_offdiag(const LevelView& L, const LeafRec& R, const Src& src, const HalfPos& p,
-                                             float* tile, typename Src::Quad& c, float xc[4], float s[4]) {
+                                             float (*tiles)[512], typename Src::Quad& c, float xc[4], float s[4]) {
     const int row = p.row, lx = row >> 3, ly = row & 7, z0 = p.z0;
     const int off = row * 8 + z0;
     // an absent neighbour leaf reads the own leaf instead and counts as 0
@@ -212,7 +213,7 @@ __device__ __forceinline__ void half_offdiag(const LevelView& L, const LeafRec& 
     for (int k = 0; k < 4; ++k) {
         have[k] = own[k] || R.nb[k] >= 0;
         const bool nb = !own[k] && R.nb[k] >= 0;
-        if (!kTile || nb)
+        if (!kTiles || nb)
             src.load(nb ? R.nb[k] : p.leaf, nb ? R.nbsd[k] : R.sd, nb ? R.nbpar[k] : R.par,
                      own[k] ? o_own[k] : o_nb[k], sq[k]);
     }
@@ -220,7 +221,10 @@ __device__ __forceinline__ void half_offdiag(const LevelView& L, const LeafRec& 
     const bool hi = z0 != 0;
     const int nz = hi ? R.nb[5] : R.nb[4];
     typename Src::One oq;
-    src.load(nz >= 0 ? nz : p.leaf, nz >= 0 ? (hi ? R.nbsd[5] : R.nbsd[4]) : R.sd,
+    // (one brick line a lane: from LDS where the workgroup holds the neighbour too)
+    const int first = kTiles > 0 ? logical_block() * kTiles : 0;
+    const bool nz_in = kTiles > 0 && nz >= first && nz < first + kTiles;
+    if (!nz_in) src.load(nz >= 0 ? nz : p.leaf, nz >= 0 ? (hi ? R.nbsd[5] : R.nbsd[4]) : R.sd,
              nz >= 0 ? (hi ? R.nbpar[5] : R.nbpar[4]) : R.par, row * 8 + (hi ? 0 : 7), oq);
     float cxm[4], cxp[4], cym[4], cyp[4], cz[4];
     const float d = L.dflt_off;
@@ -233,7 +237,8 @@ __device__ __forceinline__ void half_offdiag(const LevelView& L, const LeafRec& 
 #pragma unroll
     for (int z = 0; z < 4; ++z) xc[z] = src.value(c, z);
     float v[4][4];
-    if constexpr (kTile) {
+    if constexpr (kTiles > 0) {
+        float* tile = tiles[threadIdx.x >> 7];
         sth(tile + off, xc);
         __syncthreads();
 #pragma unroll
@@ -250,7 +255,9 @@ __device__ __forceinline__ void half_offdiag(const LevelView& L, const LeafRec& 
 #pragma unroll
             for (int z = 0; z < 4; ++z) v[k][z] = have[k] ? src.value(sq[k], z) : 0.f;
     }
-    const float zout = nz >= 0 ? src.value(oq) : 0.f;
+    float zout = nz >= 0 && !nz_in ? src.value(oq) : 0.f;
+    if constexpr (kTiles > 0)
+        if (nz_in) zout = tiles[nz - first][row * 8 + (hi ? 0 : 7)];
     const float xo = pair_swap(hi ? xc[0] : xc[3]), co = pair_swap(cz[0]);
     const float zm = hi ? xo : zout, zp = hi ? zout : xo, czp = hi ? czout : co;
 #pragma unroll
@@ -265,22 +272,33 @@ __device__ __forceinline__ void half_offdiag(const LevelView& L, const LeafRec& 
     }
 }
 
-// weighted Jacobi on the lane's voxels, 0 off the DOFs (jacobi_row, mask_row)
-__device__ __forceinline__ void half_jacobi(const LevelView& L, const LeafRec& R, const HalfPos& p, const float xc[4],
-                                            const float s[4], const float b[4], float w, uint32_t m, float y[4]) {
-    const int off = p.row * 8 + p.z0;
-    float dg[4], inv[4];
-    ldh_slot(L.diag, R.sd, off, L.dflt_diag, dg);
-    ldh_slot(L.invdiag, R.sd, off, L.dflt_invdiag, inv);
-#pragma unroll
-    for (int z = 0; z < 4; ++z) {
-        const float ax = fmaf(xc[z], dg[z], s[z]);
-        float r = b[z] - ax;
-        r = r * inv[z];
-        const float v = fmaf(w, r, xc[z]);
-        y[z] = ((m >> z) & 1u) ? v : 0.f;
+// The remaining operands of a Jacobi sweep on the lane's voxels. Loaded behind
+// the off-diagonal sum's barrier they cost a second memory latency; loaded
+// before it, registers and with them wavefronts. At 92428 leaves, behind /
+// before: the first two sweeps 149 / 143 us, the step's diagonal 270 / 258; but
+// the plain sweep 132 / 132, with its dot product 142 / 145, and the one after
+// the prolongation 180 / 211 (72 / 82 registers: six wavefronts a SIMD / five).
+struct JacobiHalf {
+    float dg[4], inv[4], b[4];
+    template <class VB>
+    __device__ __forceinline__ void load(const LevelView& L, const LeafRec& R, const HalfPos& p, const VB* B) {
+        const int off = p.row * 8 + p.z0;
+        ldh(B + size_t(p.leaf) * 512 + off, b);
+        ldh_slot(L.diag, R.sd, off, L.dflt_diag, dg);
+        ldh_slot(L.invdiag, R.sd, off, L.dflt_invdiag, inv);
     }
-}
+    // weighted Jacobi, 0 off the DOFs (jacobi_row, mask_row)
+    __device__ __forceinline__ void sweep(const float xc[4], const float s[4], float w, uint32_t m, float y[4]) const {
+#pragma unroll
+        for (int z = 0; z < 4; ++z) {
+            const float ax = fmaf(xc[z], dg[z], s[z]);
+            float r = b[z] - ax;
+            r = r * inv[z];
+            const float v = fmaf(w, r, xc[z]);
+            y[z] = ((m >> z) & 1u) ? v : 0.f;
+        }
+    }
+};
 
 }  // namespace dev
 }  // namespace uaamg
