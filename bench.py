@@ -100,7 +100,7 @@ def kernel_rooflines(lap, iterations: int, reps: int) -> list:
     mixed = lap.precision == 1
     mode0 = 6 if mixed else 2
     ms = lap.time_apply(0, mode0, reps=reps)
-    out.append({"kernel": ("apply_kernel<2, true, bf16, float, bf16>" if mixed else "apply_kernel<2, true>") +
+    out.append({"kernel": ("jacobi_half_kernel<true, bf16, float, bf16>" if mixed else "jacobi_half_kernel<true>") +
                           " (level-0 Jacobi sweep)", "bytes_per_launch": lap.algorithmic_bytes(0, mode0),
                 "ms_per_launch": ms, "launches_per_solve": 2 * W})
     vt = "bf16" if mixed else "float"
@@ -110,7 +110,7 @@ def kernel_rooflines(lap, iterations: int, reps: int) -> list:
         ms = lap.time_apply(l, 7, reps=reps)
         name = (f"block_post_cg_kernel<{vt}> (level-{l} post-visit with the level-{L - 1} coarsest CG in front)"
                 if km[l]["post_cg"] else
-                f"block_visit_kernel<3, 2, {vt}> (level-{l} post-visit: prolongation + 3 sweeps)")
+                f"block_visit_kernel<2, {vt}> (level-{l} post-visit: prolongation + 3 sweeps)")
         out.append({"kernel": name, "bytes_per_launch": lap.algorithmic_bytes(l, 7),
                     "ms_per_launch": ms, "launches_per_solve": W * 2 ** l})
     # the standalone coarsest CG runs only when the level above does not take it into its post-visit
@@ -302,8 +302,8 @@ def main() -> int:
         roofline = roofline_fp32 = roof_sweep = None
         kernels_mx = kernels_32 = []
     else:
-        roof_sweep = roof(lap_mx, 6, "apply_kernel<2, true, bf16, float, bf16> (level-0 Jacobi sweep, BF16 W-cycle)")
-        roofline_fp32 = roof(lap, 2, "apply_kernel<2, true> (level-0 weighted Jacobi sweep, FP32)")
+        roof_sweep = roof(lap_mx, 6, "jacobi_half_kernel<true, bf16, float, bf16> (level-0 Jacobi sweep, BF16 W-cycle)")
+        roofline_fp32 = roof(lap, 2, "jacobi_half_kernel<true> (level-0 weighted Jacobi sweep, FP32)")
         # the kernel that takes the most time per solve (live launch times x launches per solve)
         kernels_mx = kernel_rooflines(lap_mx, it_mx, args.kernel_reps)
         kernels_32 = kernel_rooflines(lap, it32, args.kernel_reps)
