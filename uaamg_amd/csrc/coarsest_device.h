@@ -16,14 +16,16 @@
 // with w = A z, one reduction gives ||r||^2, g = <r, z> and d = <z, w>; then
 // beta = g / g_old, <p, A p> = d - beta^2 <p, A p>_old, alpha = g / <p, A p>,
 // p = z + beta p and q = A p = w + beta q. The same vectors as Eigen's loop,
-// rounded differently. Eigen's stopping test on ||r||^2 after an update is
-// made by the next iteration's sums, before anything changes. With the sum of
+// rounded differently, for small right-hand sides too (cg_scale.h). Eigen's
+// stopping test on ||r||^2 after an update is made by the next iteration's
+// sums, before anything changes. With the sum of
 // <p, A p> kept apart (two reductions per iteration) a solve of 1697 rows took
 // 13.5 us, with one 11.9; the rows packed to 48 bytes.
 #pragma once
 
 #include <cfloat>
 
+#include "cg_scale.h"
 #include "poisson_kernels.h"
 #include "wave_reduce.h"
 
@@ -132,11 +134,24 @@ __device__ void coarsest_cg_block(const CoarsestView& C, const V* B, V* X, CgSha
             }
         }
         // the barrier also orders this step's reads of z before the writes below
-        const float3 s = cg_sum3<kRowThreads>(rr, rz, zw, sh, parity);
+        float3 s = cg_sum3<kRowThreads>(rr, rz, zw, sh, parity);
         float beta = 0.f;
         if (it == 0) {
             threshold = fmaxf(C.tol * C.tol * s.x, FLT_MIN);
             if (s.x == 0.f || s.x < threshold) break;
+            if (cg_needs_scale(s.y)) {   // the same step with c D^-1
+                const float c = cg_scale(s.y);
+                rz = zw = 0.f;
+#pragma unroll
+                for (int j = 0; j < kPer; ++j) {
+                    cf[j][7] *= c;
+                    z[j] *= c;
+                    w[j] *= c;
+                    rz = fmaf(r[j], z[j], rz);
+                    zw = fmaf(z[j], w[j], zw);
+                }
+                s = cg_sum3<kRowThreads>(0.f, rz, zw, sh, parity);
+            }
             sigma = s.z;
         } else {
             if (s.x < threshold) break;

@@ -6,13 +6,15 @@
 // Each thread keeps up to kPer rows in registers (15 values, 15 column
 // offsets as 16-bit pairs) and only z is shared, so an iteration touches LDS
 // alone; the form with one sum over the block per iteration is the one of
-// coarsest_device.h (Chronopoulos and Gear). A row's padding multiplies the
+// coarsest_device.h (Chronopoulos and Gear), for small right-hand sides with a
+// factor of the preconditioner (cg_scale.h). A row's padding multiplies the
 // shared vector's last slot, which holds zero. With the rows streamed from
 // memory in every iteration a system of more than 1024 rows took 52 us.
 #pragma once
 
 #include <cfloat>
 
+#include "cg_scale.h"
 #include "viscosity_kernels.h"
 #include "wave_reduce.h"
 
@@ -24,6 +26,28 @@ constexpr int kVCgThreads = 512;
 struct ViscCgShared {
     float4 red[2][kVCgThreads / 64];
 };
+
+// Sums (a, b, c) over the row threads with one barrier (cg_sum3).
+__device__ __forceinline__ float3 visc_cg_sum3(float a, float b, float c, ViscCgShared& sh, int& par) {
+    const int w = threadIdx.x >> 6;
+    if (w < kVCgThreads / 64) {
+        a = wave_sum_dpp(a);
+        b = wave_sum_dpp(b);
+        c = wave_sum_dpp(c);
+        if ((threadIdx.x & 63) == 0) sh.red[par][w] = make_float4(a, b, c, 0.f);
+    }
+    __syncthreads();
+    float3 s = make_float3(0.f, 0.f, 0.f);
+#pragma unroll
+    for (int i = 0; i < kVCgThreads / 64; ++i) {
+        const float4 v = sh.red[par][i];
+        s.x += v.x;
+        s.y += v.y;
+        s.z += v.z;
+    }
+    par ^= 1;
+    return s;
+}
 
 // Solves the system for the right-hand side ld(d) and hands the solution to
 // st(d, x); sz has room for C.n + 1 floats. Row d belongs to thread d %
@@ -91,26 +115,25 @@ __device__ __forceinline__ void visc_cg_block(const ViscCoarsestView& C, float* 
                 zw = fmaf(z, t, zw);
             }
         }
-        if ((tid >> 6) < kVCgThreads / 64) {
-            rr = wave_sum_dpp(rr);
-            rz = wave_sum_dpp(rz);
-            zw = wave_sum_dpp(zw);
-            if ((tid & 63) == 0) sh.red[par][tid >> 6] = make_float4(rr, rz, zw, 0.f);
-        }
-        __syncthreads();   // also orders this step's reads of z before the writes below
-        float3 s = make_float3(0.f, 0.f, 0.f);
-#pragma unroll
-        for (int i = 0; i < kVCgThreads / 64; ++i) {
-            const float4 v = sh.red[par][i];
-            s.x += v.x;
-            s.y += v.y;
-            s.z += v.z;
-        }
-        par ^= 1;
+        // the barrier also orders this step's reads of z before the writes below
+        float3 s = visc_cg_sum3(rr, rz, zw, sh, par);
         float beta = 0.f;
         if (it == 0) {
             threshold = fmaxf(C.tol * C.tol * s.x, FLT_MIN);
             if (s.x == 0.f || s.x < threshold) break;
+            if (cg_needs_scale(s.y)) {   // the same step with c D^-1
+                const float c = cg_scale(s.y);
+                rz = zw = 0.f;
+#pragma unroll
+                for (int j = 0; j < kPer; ++j) {
+                    inv[j] *= c;
+                    w[j] *= c;
+                    const float z = inv[j] * r[j];
+                    rz = fmaf(r[j], z, rz);
+                    zw = fmaf(z, w[j], zw);
+                }
+                s = visc_cg_sum3(0.f, rz, zw, sh, par);
+            }
             sigma = s.z;
         } else {
             if (s.x < threshold) break;
