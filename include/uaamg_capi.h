@@ -249,7 +249,9 @@ typedef struct uaamg_face_channel {
  * velocity elsewhere (the reference's deep copy), reflected the reflected velocity likewise; the
  * active masks end as the updated faces. pressure_dev: the solve's DOF-ordered result (device).
  * Replaces FLIP_Solver_OpenVDB::apply_pressure_gradient (FLIP_vdb.cpp:2571-2667); bit-identical to
- * its restatement. channels: 3 entries (x, y, z); solid_velocity may be NULL (zero).
+ * its restatement. channels: 3 entries (x, y, z), updated in that order: where channels share an
+ * array, the later one finds what the earlier one left in it (shared active masks narrow from
+ * channel to channel). solid_velocity may be NULL (zero).
  */
 int uaamg_poisson_apply_pressure_gradient_device(uaamg_poisson* h, const float* pressure_dev,
                                                  const uaamg_grid* liquid_phi, const uaamg_grid* face_weights,

@@ -119,9 +119,23 @@ int apply_pressure_gradient_device(PoissonDevice& d, const float* pressure_dev, 
         for (DevBuf* b : {&vel_b, &upd_b, &refl_b}) b->release();
         return 0;
     };
+    // A channel's masks are read after those of the channels before it are written, where the arrays overlap.
+    int pending = 0;   // first channel whose masks are still to be downloaded
+    auto shares_masks = [&](int c) {
+        auto first = [&](int k) { return reinterpret_cast<uintptr_t>(channels[k].active); };
+        auto end = [&](int k) { return first(k) + size_t(channels[k].nleaf) * 8 * sizeof(uint64_t); };
+        for (int k = pending; k < c; ++k)
+            if (first(k) < end(c) && first(c) < end(k)) return true;
+        return false;
+    };
     for (int c = 0; c < 3; ++c) {
         FaceChannelRef& ch = channels[c];
         if (ch.nleaf == 0) continue;
+        if (values_on_device && shares_masks(c)) {
+            for (; pending < c; ++pending)
+                if (int rc = download(pending)) return rc;
+            if (hipError_t e = hipStreamSynchronize(s)) return hip_fail(e, "pressure gradient sync");
+        }
         int32_t* const tab_d = tab_at(c);
         uint64_t* const act_d = act_at(c);
         const size_t n = size_t(ch.nleaf);
@@ -179,8 +193,8 @@ int apply_pressure_gradient_device(PoissonDevice& d, const float* pressure_dev, 
     }
     // values on the device: a channel's masks are uploaded beside the kernel of the one before
     if (values_on_device)
-        for (int c = 0; c < 3; ++c)
-            if (int rc = download(c)) return rc;
+        for (; pending < 3; ++pending)
+            if (int rc = download(pending)) return rc;
     if (hipError_t e = hipStreamSynchronize(s)) return hip_fail(e, "pressure gradient sync");
     return 0;
 }
