@@ -58,3 +58,34 @@ def test_noalloc_rhs_matches_the_allocating_build(hip_available, sizes):
         host = lap.createPressurePoissonRightHandSide(s.weights, s.vx, s.vy, s.vz)
         assert np.array_equal(out.cpu().numpy(), host)
         del keep
+
+
+@pytest.mark.parametrize("kind", ["matched", "misaligned", "duplicate"])
+def test_noalloc_matches_leaves_on_the_host(hip_available, kind):
+    """Leaves in any order with some missing; and refused origins, with nothing written. Each grid goes
+    into one host table, which serves the check and the matching."""
+    import torch
+    noalloc, _ = _bind()
+    _say(f"[case] noalloc leaves {kind}")
+    s = U.Scene(0, 48, seed=2)
+    lap = U.LaplacianWithLevel(s.phi, s.weights, dt=1.0, dx=s.dx)
+    rng = np.random.default_rng(3)
+    grids = [s.weights]
+    for g in (s.vx, s.vy, s.vz):
+        p = rng.permutation(g.origins.shape[0])[:-5]
+        grids.append(U.Grid(g.origins[p].copy(), g.values[p].copy(), None, (0.25, 0.25, 0.25)))
+    org = grids[2].origins
+    if kind != "matched":
+        org[-1] = org[0] if kind == "duplicate" else org[-1] + 1
+    vals = [torch.from_numpy(np.ascontiguousarray(g.values, np.float32)).to("cuda:0") for g in grids]
+    st = [g._struct(v.data_ptr()) for g, v in zip(grids, vals)]
+    out = torch.full((lap.mNumDof,), 7.0, device="cuda:0")
+    torch.cuda.synchronize()
+    rc = noalloc(lap._h, *[C.byref(x) for x in st], None, C.c_void_p(out.data_ptr()))
+    torch.cuda.synchronize()
+    if kind == "matched":
+        assert rc == 0
+        assert np.array_equal(out.cpu().numpy(), lap.createPressurePoissonRightHandSide(*grids))
+    else:
+        assert rc < 0 and (b"duplicate" if kind == "duplicate" else b"multiple of 8") in U.lib().uaamg_last_error()
+        assert bool((out == 7.0).all())

@@ -72,7 +72,7 @@ hipError_t LeafMatch::query(int from, const std::vector<MatchColumn>& cols, int3
     return launch_match_query(sets_, q, s);
 }
 
-bool bad_origins(int64_t n, const int32_t* origins, bool* misaligned) {
+bool bad_origins(int64_t n, const int32_t* origins, LeafLookup& lookup, bool* misaligned) {
     std::vector<Coord> o(static_cast<size_t>(n));
     for (int64_t i = 0; i < n; ++i) {
         o[size_t(i)] = {origins[3 * i], origins[3 * i + 1], origins[3 * i + 2]};
@@ -82,11 +82,15 @@ bool bad_origins(int64_t n, const int32_t* origins, bool* misaligned) {
         }
     }
     *misaligned = false;
-    LeafLookup lookup;
     lookup.build(o);
     for (size_t i = 0; i < o.size(); ++i)
         if (lookup.find(o[i]) != int32_t(i)) return true;
     return false;
+}
+
+bool bad_origins(int64_t n, const int32_t* origins, bool* misaligned) {
+    LeafLookup lookup;
+    return bad_origins(n, origins, lookup, misaligned);
 }
 
 }  // namespace uaamg

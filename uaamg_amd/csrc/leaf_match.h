@@ -16,6 +16,8 @@
 
 namespace uaamg {
 
+class LeafLookup;
+
 constexpr int kMatchSets = 8;    // different sets of origins of one call
 constexpr int kMatchCols = 20;   // columns of one query
 
@@ -69,7 +71,9 @@ private:
     MatchSets sets_{};
 };
 
-// The refusal of a grid's origins (misaligned, then duplicate), or false
+// The refusal of a grid's origins (misaligned, then duplicate), or false with
+// the grid's lookup built
+bool bad_origins(int64_t n, const int32_t* origins, LeafLookup& lookup, bool* misaligned);
 bool bad_origins(int64_t n, const int32_t* origins, bool* misaligned);
 
 }  // namespace uaamg

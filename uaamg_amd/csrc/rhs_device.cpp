@@ -90,12 +90,8 @@ int build_rhs_impl(PoissonDevice& d, const RhsGridRef* grids, float* rhs_dof, in
         const RhsGridRef& r = grids[g];
         if (tab_scratch) {
             bool misaligned;
-            if (bad_origins(r.nleaf, r.origins, &misaligned)) return refusal(misaligned);
-            std::vector<Coord> org(size_t(r.nleaf));
-            for (size_t i = 0; i < org.size(); ++i)
-                org[i] = {r.origins[3 * i], r.origins[3 * i + 1], r.origins[3 * i + 2]};
             LeafLookup lookup;
-            lookup.build(org);
+            if (bad_origins(r.nleaf, r.origins, lookup, &misaligned)) return refusal(misaligned);
             for (size_t i = 0; i < n0; ++i) {
                 const Coord o = l0.origin[i];
                 const Coord at[4] = {o, {o.x + 8, o.y, o.z}, {o.x, o.y + 8, o.z}, {o.x, o.y, o.z + 8}};
