@@ -38,10 +38,9 @@ struct ViscRowsView {
 constexpr int64_t kViscRowsMax = 20480;
 
 // Threads of a visit's workgroup and rows per step: 1024 where the coarsest
-// rows fit 128 registers a thread (two of them), 512 beyond. Steps of one launch
-// have one size, so a batch goes by its largest coarsest level.
+// rows fit 128 registers a thread (two of them), 512 beyond.
 constexpr int kViscRowsWideNc = 1024;
-inline int visc_rows_step(int max_nc) { return max_nc <= kViscRowsWideNc ? 1024 : 512; }
+inline int visc_rows_step(int nc) { return nc <= kViscRowsWideNc ? 1024 : 512; }
 
 // A step is up to that many rows of one group: {first row, the group's end,
 // plus kViscStepLast on a pass's last step (a barrier follows)}.
@@ -63,11 +62,10 @@ hipError_t launch_visc_rows_build(const ViscLevelView& F, const ViscLevelView& C
 
 // nvisits visits of the level (the first from a zero guess when precon, else
 // from x), with right-hand side b and the coarsest solves inside; the result
-// goes to x. One workgroup per problem, `count` of them: views and cviews are
-// device arrays, max_n and max_nc the problems' largest sizes.
-hipError_t launch_visc_rows_visit(const ViscRowsView* views, const ViscCoarsestView* cviews, int count, int max_n,
-                                  int max_nc, const float* b, float* x, bool precon, int nvisits, hipStream_t s);
-hipError_t launch_visc_rows_visit(const ViscRowsView* views, const ViscCoarsestView* cviews, int count, int max_n,
-                                  int max_nc, const bf16* b, bf16* x, bool precon, int nvisits, hipStream_t s);
+// goes to x. view (of n rows) and cview (of nc) are in device memory.
+hipError_t launch_visc_rows_visit(const ViscRowsView* view, const ViscCoarsestView* cview, int n, int nc,
+                                  const float* b, float* x, bool precon, int nvisits, hipStream_t s);
+hipError_t launch_visc_rows_visit(const ViscRowsView* view, const ViscCoarsestView* cview, int n, int nc,
+                                  const bf16* b, bf16* x, bool precon, int nvisits, hipStream_t s);
 
 }  // namespace uaamg

@@ -341,31 +341,29 @@ __device__ __forceinline__ void rows_visit(const ViscRowsView& R, const ViscCoar
     for (int row = tid; row < R.n; row += kT) st1v(X + gload<int>(R.pos, uint32_t(row) * 4u), xs[row]);
 }
 
-// workgroup i: problem i
+// one workgroup
 template <class V, int kPer, int kT>
-__global__ __launch_bounds__(kT) void visc_rows_visit_kernel(const ViscRowsView* views, const ViscCoarsestView* cviews,
+__global__ __launch_bounds__(kT) void visc_rows_visit_kernel(const ViscRowsView* view, const ViscCoarsestView* cview,
                                                              const V* B, V* X, int precon, int nvisits) {
-    const ViscRowsView R = views[blockIdx.x];
-    const ViscCoarsestView C = cviews[blockIdx.x];
+    const ViscRowsView R = *view;
+    const ViscCoarsestView C = *cview;
     rows_visit<V, kPer, kT>(R, C, B, X, precon != 0, nvisits);
 }
 
 template <class V>
-hipError_t visit(const ViscRowsView* views, const ViscCoarsestView* cviews, int count, int max_n, int max_nc,
-                 const V* b, V* x, bool precon, int nvisits, hipStream_t s) {
-    if (count <= 0) return hipSuccess;
-    if (max_n <= 0 || max_n > kViscRowsMax || max_nc <= 0 || max_nc > kViscMaxCoarsest || nvisits < 1)
-        return hipErrorInvalidValue;
-    const size_t lds = (size_t(max_n) + size_t(max_nc) + 2) * sizeof(float);
-    const unsigned g = unsigned(count);
+hipError_t visit(const ViscRowsView* view, const ViscCoarsestView* cview, int n, int nc, const V* b, V* x, bool precon,
+                 int nvisits, hipStream_t s) {
+    if (n <= 0 || n > kViscRowsMax || nc <= 0 || nc > kViscMaxCoarsest || nvisits < 1) return hipErrorInvalidValue;
+    const size_t lds = (size_t(n) + size_t(nc) + 2) * sizeof(float);
     const int p = precon ? 1 : 0;
+    // (the steps of the view are cut for the same thread count)
     static_assert(2 * kVCgThreads == kViscRowsWideNc, "the wide form's coarsest size");
-    if (visc_rows_step(max_nc) == 1024)
-        visc_rows_visit_kernel<V, 2, 1024><<<g, 1024, lds, s>>>(views, cviews, b, x, p, nvisits);
-    else if (max_nc <= 4 * kVCgThreads)
-        visc_rows_visit_kernel<V, 4, 512><<<g, 512, lds, s>>>(views, cviews, b, x, p, nvisits);
+    if (visc_rows_step(nc) == 1024)
+        visc_rows_visit_kernel<V, 2, 1024><<<1, 1024, lds, s>>>(view, cview, b, x, p, nvisits);
+    else if (nc <= 4 * kVCgThreads)
+        visc_rows_visit_kernel<V, 4, 512><<<1, 512, lds, s>>>(view, cview, b, x, p, nvisits);
     else
-        visc_rows_visit_kernel<V, 8, 512><<<g, 512, lds, s>>>(views, cviews, b, x, p, nvisits);
+        visc_rows_visit_kernel<V, 8, 512><<<1, 512, lds, s>>>(view, cview, b, x, p, nvisits);
     return hipGetLastError();
 }
 
@@ -404,13 +402,13 @@ hipError_t launch_visc_rows_build(const ViscLevelView& F, const ViscLevelView& C
     return hipGetLastError();
 }
 
-hipError_t launch_visc_rows_visit(const ViscRowsView* views, const ViscCoarsestView* cviews, int count, int max_n,
-                                  int max_nc, const float* b, float* x, bool precon, int nvisits, hipStream_t s) {
-    return visit<float>(views, cviews, count, max_n, max_nc, b, x, precon, nvisits, s);
+hipError_t launch_visc_rows_visit(const ViscRowsView* view, const ViscCoarsestView* cview, int n, int nc,
+                                  const float* b, float* x, bool precon, int nvisits, hipStream_t s) {
+    return visit<float>(view, cview, n, nc, b, x, precon, nvisits, s);
 }
-hipError_t launch_visc_rows_visit(const ViscRowsView* views, const ViscCoarsestView* cviews, int count, int max_n,
-                                  int max_nc, const bf16* b, bf16* x, bool precon, int nvisits, hipStream_t s) {
-    return visit<bf16>(views, cviews, count, max_n, max_nc, b, x, precon, nvisits, s);
+hipError_t launch_visc_rows_visit(const ViscRowsView* view, const ViscCoarsestView* cview, int n, int nc,
+                                  const bf16* b, bf16* x, bool precon, int nvisits, hipStream_t s) {
+    return visit<bf16>(view, cview, n, nc, b, x, precon, nvisits, s);
 }
 
 }  // namespace uaamg

@@ -551,15 +551,15 @@ void ViscDevice::rbgs(int level, V* x, const V* b, bool xyz) {
     }
 }
 
-// simd_viscosity3d::mucycle (:3828-3884) with mu = 2, n = 2. At the level
-// above the coarsest the second visit would solve the same right-hand side
-// from zero again (solve_exact starts from a zero guess) and is skipped.
 template <class V>
 void ViscDevice::rows_visit(V* x, const V* b, bool precon, int nvisits) {
-    check(launch_visc_rows_visit(rows_dev_, cv_dev_, 1, rows_.n, rows_.nc, b, x, precon, nvisits, stream_),
+    check(launch_visc_rows_visit(rows_dev_, cv_dev_, rows_.n, rows_.nc, b, x, precon, nvisits, stream_),
           "rows visit");
 }
 
+// simd_viscosity3d::mucycle (:3828-3884) with mu = 2, n = 2. At the level
+// above the coarsest the second visit would solve the same right-hand side
+// from zero again (solve_exact starts from a zero guess) and is skipped.
 template <class V>
 void ViscDevice::mucycle(int level, V* x, const V* b, bool precon) {
     const int L = int(lv_.size());
