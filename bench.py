@@ -436,6 +436,17 @@ def main() -> int:
     return 0
 
 
+def median_ms(fn, reps: int = 9) -> float:
+    """Median of calls that return with their work done. (Not a mean of a few: the HIP runtime stalls
+    one copy among a process's first for about 6 ms.)"""
+    ts = []
+    for _ in range(reps):
+        t0 = time.perf_counter()
+        fn()
+        ts.append(time.perf_counter() - t0)
+    return 1e3 * sorted(ts)[reps // 2]
+
+
 def rhs_build(lap, scene, b_host, t_host_s: float, dev) -> dict:
     """The right-hand side built on the host (uaamg_poisson_build_rhs) and on the
     device (uaamg_poisson_build_rhs_device) from host-resident grids (values
@@ -447,14 +458,10 @@ def rhs_build(lap, scene, b_host, t_host_s: float, dev) -> dict:
     grids = [scene.weights, scene.vx, scene.vy, scene.vz]
     out = torch.empty(lap.mNumDof, dtype=torch.float32, device=dev)
 
-    def timed(fn, reps=3):
+    def timed(fn):
         fn()
         torch.cuda.synchronize()
-        t0 = time.perf_counter()
-        for _ in range(reps):
-            fn()
-        torch.cuda.synchronize()
-        return 1e3 * (time.perf_counter() - t0) / reps
+        return median_ms(fn)
 
     ms_upload = timed(lambda: lap.createPressurePoissonRightHandSide_device(out.data_ptr(), *grids))
     same_upload = bool(np.array_equal(out.cpu().numpy(), b_host))
@@ -525,12 +532,7 @@ def pressure_gradient(lap, scene, pressure) -> dict:
             raise RuntimeError(f"pressure gradient returned {rc}")
     call()
     torch.cuda.synchronize()
-    reps = 5
-    t0 = time.perf_counter()
-    for _ in range(reps):
-        call()
-    torch.cuda.synchronize()
-    ms_dev = 1e3 * (time.perf_counter() - t0) / reps
+    ms_dev = median_ms(call)
     del keep
     return {"ms_per_call": round(ms, 2), "faces_updated": faces, "velocity_mb": round(mb, 1),
             "io": "velocity, update and reflected grids through host memory",

@@ -193,13 +193,16 @@ int uaamg_poisson_build_rhs(const uaamg_poisson* h, const uaamg_grid* face_weigh
 
 /*
  * The same right-hand side built on the device into rhs_dev (ndof floats, DOF order, device memory),
- * bit-identical to uaamg_poisson_build_rhs: one wavefront per level-0 DOF leaf reads the face weights,
- * liquid and solid velocities at each DOF voxel and at its +x/+y/+z neighbour voxel. The grids' leaves
- * are matched to the DOF leaves by origin on the host (leaf tables, O(leaves)); values_on_device = 0:
- * each grid's values are host memory, uploaded for the call; 1: they are device memory
- * ([nleaf][512][ncomp] in the grid's own leaf order; origins stay host memory). solid_velocity may be
- * NULL (zero). Allocates device memory for the call (values when uploaded, the leaf tables) and
- * returns after rhs_dev is written.
+ * bit-identical to uaamg_poisson_build_rhs: the face weights, liquid and solid velocities are read at
+ * each DOF voxel and at its +x/+y/+z neighbour voxel, a wavefront per x-plane of a level-0 DOF leaf.
+ * The grids' leaves are matched to the DOF leaves by origin on the device. values_on_device = 0: each
+ * grid's values are host memory, uploaded for the call (device memory of their size, freed on return);
+ * 1: they are device memory ([nleaf][512][ncomp] in the grid's own leaf order; origins stay host
+ * memory). solid_velocity may be NULL (zero). Returns after rhs_dev is written.
+ * The matching uses scratch memory that the handle keeps until it gives up its device memory, and that
+ * grows with the largest call: 80 bytes per level-0 DOF leaf, and 36 to 60 per leaf of each grid whose
+ * origins differ from the others' (uaamg_poisson_apply_pressure_gradient_device shares it: 264 per
+ * leaf of the largest velocity channel in the place of the 80).
  * Replaces LaplacianWithLevel::createPressurePoissonRightHandSide (simd_vdb_poisson.h:59-65, .cpp:101-127)
  * for callers whose velocities live on the GPU, or whose host cannot afford the per-voxel loop.
  */
@@ -214,7 +217,7 @@ int uaamg_poisson_build_rhs_device(uaamg_poisson* h, const uaamg_grid* face_weig
  * uaamg_poisson_build_rhs_device with no device allocation (no counterpart in the reference): for
  * callers that cannot allocate device memory - code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc. Every grid's values must already be device memory (as with
- * values_on_device = 1); the leaf tables go into a fixed scratch array of the library (10 MiB per
+ * values_on_device = 1); the leaf tables are made on the host and go into a fixed scratch array of the library (10 MiB per
  * GPU, held until the process ends) instead of a per-call allocation. Returns UAAMG_EINVAL when
  * level 0 has more than UAAMG_RHS_NOALLOC_MAX_LEAVES DOF leaves. All calls on one GPU share that
  * array: calls that overlap on one GPU (several host threads) race on it and must be serialised by

@@ -33,9 +33,10 @@ __device__ __forceinline__ bool pressure_at(const GradArgs& a, const DofPlane& d
 
 // One wavefront per x-plane of a velocity leaf, a lane per voxel: every access
 // to a vector is consecutive, the plane's masks are one word, and a lane's
-// loads do not wait for each other. Bound by HBM (reads of phi, the weights
-// and the pressure, three writes): 72 us a channel at 13115 leaves, where
-// a lane per z-row stepping through its eight voxels took 326.
+// loads do not wait for each other. 72 us a channel at 13115 leaves, where a
+// lane per z-row stepping through its eight voxels took 326. 240 MB pass
+// through HBM (every channel reads the weights' three components), 3.3 TB/s,
+// two thirds of a copy's rate; a wavefront waits for three quarters of its life.
 __global__ __launch_bounds__(kBlockThreads) void pressure_gradient_kernel(int64_t nleaf, GradArgs a, uint64_t* active,
                                                                           float* vel, float* upd, float* refl) {
     const int gw = __builtin_amdgcn_readfirstlane(logical_block() * kWavesPerBlock + int(threadIdx.x >> 6));

@@ -51,8 +51,9 @@ struct RhsGridRef {
 
 class PoissonDevice;
 
-// Matches the leaves on the device (leaf_match.h), uploads host-resident
-// values for the call, and runs the kernel on the solver's stream; returns when rhs_dof is written. grids: kRhsGrids entries
+// Matches the leaves on the device (leaf_match.h) in the handle's scratch
+// memory, uploads host-resident values for the call, and runs the kernel on the
+// solver's stream; returns when rhs_dof is written. grids: kRhsGrids entries
 // in kRhs* order (an empty solid-velocity grid reads its background).
 // Returns 0, or a negative uaamg status with err set.
 int build_poisson_rhs_device(PoissonDevice& d, const RhsGridRef* grids, float* rhs_dof, std::string& err);
@@ -63,8 +64,8 @@ constexpr int64_t kRhsNoAllocMaxLeaves = 131072;
 
 // The same build with no device allocation: every grid's values must already
 // be device memory, and the leaf tables are matched on the host (the sets of a
-// match on the device have no bound that a fixed array could meet) and go into the library's fixed per-device
-// scratch array, which all calls on one GPU share (calls that overlap on one
+// match on the device have no bound that a fixed array could meet) and go into
+// the library's fixed per-device scratch array, which all calls on one GPU share (calls that overlap on one
 // GPU race on it). Returns 0, or a negative uaamg status with err set.
 int build_poisson_rhs_device_noalloc(PoissonDevice& d, const RhsGridRef* grids, float* rhs_dof, std::string& err);
 

@@ -12,9 +12,12 @@ __device__ __forceinline__ float grid_value(const RhsGridDev& g, int32_t leaf, i
 }
 
 // One wavefront per x-plane of a level-0 DOF leaf, a lane per voxel (the term
-// order of BuildPoissonRhs::operator(), simd_vdb_poisson.cpp:43-84). Bound by
-// HBM: 75 us at 12193 leaves; a lane per z-row, whose voxels lie 32 and 96
-// bytes from the next lane's, took 320.
+// order of BuildPoissonRhs::operator(), simd_vdb_poisson.cpp:43-84). 76 us at
+// 12193 leaves, where a lane per z-row, whose voxels lie 32 and 96 bytes from
+// the next lane's, took 320. 173 MB pass through HBM, 2.3 TB/s, under half of a
+// copy's rate: what bounds it is latency, with three quarters of a wavefront's
+// life spent waiting for its chain of leaf table, operands (the weights at a
+// stride of 12 bytes) and store.
 __global__ __launch_bounds__(kBlockThreads) void poisson_rhs_kernel(LevelView L, RhsArgs a, float* out) {
     const int gw = __builtin_amdgcn_readfirstlane(logical_block() * kWavesPerBlock + int(threadIdx.x >> 6));
     const int leaf = gw >> 3, lx = gw & 7;
